@@ -64,9 +64,13 @@ template <typename F>
 __device__ __forceinline__ void walk_neighbours(const StepConsts& C, int i, float4 p, const float4* __restrict__ pos,
                                                 const uint32_t* __restrict__ cs, const ListEntry* __restrict__ nl,
                                                 const uint32_t* __restrict__ nn, F&& f) {
-    const uint32_t cnt = nn[i];
-    if (cnt <= (uint32_t)kListCap) {
-        for (uint32_t t = 0; t < cnt; ++t) f(list_decode(nl[list_at(C.n, i, t)], i));
+    const uint32_t head = nn[i];
+    if (head <= (uint32_t)kListCap) {
+        for (uint32_t t = 0; t < head; ++t) f(list_decode(nl[list_at(C.n, i, t)], i));
+    } else if (head & kSeqList) {
+        const uint32_t cnt = list_count(head);
+        SeqWalk at(head, i);
+        for (uint32_t t = 0; t < cnt; ++t) f(at.next(nl[list_at(C.n, i, t)]));
     } else {
         for_each_candidate(p.x, p.y, p.z, C, cs, [&](uint32_t k) {
             const float4 q = pos[k];

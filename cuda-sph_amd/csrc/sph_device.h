@@ -503,9 +503,41 @@ __device__ __forceinline__ uint32_t finish_particle(const StepConsts& C, int i, 
     return hash_particle<SLOT_KEYS>(C, pp.x, pp.y, pp.z, pid, (uint32_t)i, keyI, valI, flags);
 }
 
-// Neighbour-list entries (ListEntry): the neighbour's index relative to the particle's own.
-// Layout: slots t and t + 1 (t even) of particle i share the 32-bit word (t / 2) * n + i, so
-// a lane reads two slots per load and consecutive particles' words are contiguous.
+// Neighbour lists.  Slots t and t + 1 (t even) of particle i share the 32-bit word (t / 2) * n
+// + i, so a lane reads two slots per load and consecutive particles' words are contiguous.  A
+// slot holds the low 16 bits of the neighbour's cell-ordered index minus the particle's own;
+// the word nn[i] says how they are completed:
+//   <= kListCap   the count; every neighbour lies within [i - 2^15, i + 2^15), so any slot can
+//                 be decoded by itself (list_decode).
+//   kSeqList set  built with one lane per particle where neighbours lie farther: the count in the
+//                 low kSeqCountBits bits, above them how far before i its first candidate lies.
+//                 Indices increase along the list by less than 2^16 from one neighbour to the
+//                 next, so a walk from the first candidate on restores them (SeqWalk).  A 4.2M
+//                 particle dam break, whose layers of cells hold 33,000 particles each, left
+//                 its particles to a rescan without this: force 1,115 us per launch.
+//   else          no list: the particle's candidates are scanned again, by a reader with several
+//                 lanes per particle also in place of a kSeqList walk.
+constexpr uint32_t kSeqList = 0x80000000u;
+constexpr uint32_t kNoList = 0x7fffffffu;
+constexpr int kSeqCountBits = 10;
+constexpr uint32_t kSeqMaxBack = 1u << (31 - kSeqCountBits);
+constexpr uint32_t kListWindow = 1u << 15;
+static_assert(kListCap < (1 << kSeqCountBits), "the count fits its field");
+__device__ __forceinline__ uint32_t seq_head(uint32_t cnt, uint32_t back) {
+    return kSeqList | (back << kSeqCountBits) | cnt;
+}
+__device__ __forceinline__ uint32_t list_count(uint32_t head) { return head & ((1u << kSeqCountBits) - 1u); }
+// The neighbours of a kSeqList list in order: each is the next index after the last whose
+// offset from i has the slot's low 16 bits.
+struct SeqWalk {
+    uint32_t d;  // offset of the last neighbour; at first, of the first candidate
+    int i;
+    __device__ __forceinline__ SeqWalk(uint32_t head, int i_) : d(0u - ((head & ~kSeqList) >> kSeqCountBits)), i(i_) {}
+    __device__ __forceinline__ uint32_t next(uint32_t e) {
+        d += (uint32_t)(uint16_t)(e - d);
+        return (uint32_t)i + d;
+    }
+};
 __device__ __forceinline__ ListEntry list_encode(uint32_t k, int i) { return (ListEntry)(uint16_t)((int)k - i); }
 __device__ __forceinline__ uint32_t list_decode(ListEntry e, int i) { return (uint32_t)(i + (int)(int16_t)e); }
 __device__ __forceinline__ size_t list_at(int n, int i, uint32_t t) {
@@ -556,11 +588,12 @@ __device__ __forceinline__ PairSums naive_pair_sums(const StepConsts& C, int i, 
     const __amdgpu_buffer_rsrc_t rpos = make_rsrc(pos, (uint32_t)n * 16u);
     const __amdgpu_buffer_rsrc_t rvel = make_rsrc(vel, (uint32_t)n * 16u);
     PairSums S;
-    const uint32_t cnt = nn[i];
-    if (cnt <= (uint32_t)kListCap) {
-        // two slots per 32-bit load (list_at); the next four slots are loaded while this
-        // group's neighbours are gathered, so each group waits on one memory latency
-        static_assert(kForceUnroll == 4, "the force pass walks the list four slots at a time");
+    const uint32_t head = nn[i];
+    const uint32_t cnt = list_count(head);
+    // two slots per 32-bit load (list_at); the next four slots are loaded while this group's
+    // neighbours are gathered, so each group waits on one memory latency
+    static_assert(kForceUnroll == 4, "the force pass walks the list four slots at a time");
+    auto walk = [&](auto&& decode) {
         const uint32_t* words = reinterpret_cast<const uint32_t*>(nl) + i;
         const size_t stride = (size_t)n;
         uint32_t t = 0;
@@ -576,8 +609,11 @@ __device__ __forceinline__ PairSums naive_pair_sums(const StepConsts& C, int i, 
                 wn0 = words[0];
                 wn1 = words[stride];
             }
-            const uint32_t k[4] = {list_decode((ListEntry)w0, i), list_decode((ListEntry)(w0 >> 16), i),
-                                   list_decode((ListEntry)w1, i), list_decode((ListEntry)(w1 >> 16), i)};
+            uint32_t k[4];
+            k[0] = decode(w0);
+            k[1] = decode(w0 >> 16);
+            k[2] = decode(w1);
+            k[3] = decode(w1 >> 16);
             float4 q[4], w[4];
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
@@ -590,13 +626,19 @@ __device__ __forceinline__ PairSums naive_pair_sums(const StepConsts& C, int i, 
         for (; t < cnt; t += 2u) {  // the last one to three slots, a word at a time
             const uint32_t wd = words[0];
             words += stride;
-            const uint32_t k0 = list_decode((ListEntry)wd, i);
+            const uint32_t k0 = decode(wd);
             S.add(C, p, v, ld_f4(rpos, k0 * 16u), ld_f4(rvel, k0 * 16u), k0 == (uint32_t)i);
             if (t + 1u < cnt) {
-                const uint32_t k1 = list_decode((ListEntry)(wd >> 16), i);
+                const uint32_t k1 = decode(wd >> 16);
                 S.add(C, p, v, ld_f4(rpos, k1 * 16u), ld_f4(rvel, k1 * 16u), k1 == (uint32_t)i);
             }
         }
+    };
+    if (head <= (uint32_t)kListCap) {
+        walk([&](uint32_t e) { return list_decode((ListEntry)e, i); });
+    } else if (head & kSeqList) {
+        SeqWalk at(head, i);
+        walk([&](uint32_t e) { return at.next(e); });
     } else {
         for_each_candidate(p.x, p.y, p.z, C, cs, [&](uint32_t k) {
             const float4 q = pos[k];

@@ -27,9 +27,10 @@
 //                         The density pass appends a particle's first 32 L entries (L lanes
 //                         per particle, at most 96) to its place in its wavefront's LDS band
 //                         and copies them out slot by slot at the end (every store coalesced);
-//                         hits beyond that go straight to HBM.  nn > 96 marks a
-//                         particle whose neighbours the force pass rescans (more than 96, or
-//                         one farther than an int16 offset).
+//                         hits beyond that go straight to HBM.  nn holds the count, or
+//                         how a list with neighbours beyond the int16 window is walked, or
+//                         marks a particle whose neighbours the force pass rescans (more than
+//                         96, or out of the list's reach); see list_decode, SeqWalk
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -57,8 +58,8 @@ constexpr int kFlagOutOfGrid = 1;   // VOXEL: a finite position of this step's s
                                     // cleared by the first pass of the sort)
 
 // NAIVE neighbour-list entry: the neighbour's cell-ordered index minus the particle's own, as
-// int16 (neighbours in space are near each other in cell order).  A particle with a
-// neighbour farther away than that in cell order is marked for a rescan instead.
+// int16 (neighbours in space are near each other in cell order).  With a neighbour farther
+// away than that, the list is walked in order or the particle marked for a rescan instead.
 typedef uint16_t ListEntry;
 
 // Everything a step kernel needs, passed by value (fits the kernel-argument segment).
@@ -156,7 +157,7 @@ struct Buffers {
     float4 *dbgP, *dbgV, *dbgF;
     int32_t* nbr;          // VOXEL formulation neighbour lists, N x (1 + 32)
     ListEntry* nl;         // NAIVE neighbour lists, column-major [kListCap][N] (index offsets, self included)
-    uint32_t* nn;          // NAIVE neighbour count per cell-ordered particle (may exceed kListCap)
+    uint32_t* nn;          // NAIVE list word per cell-ordered particle (count, kSeqList or kNoList)
     double* diag_partials;
     uint32_t* flags;       // kFlagNonFinite, kFlagOutOfGrid (16 words)
     PipeTable* pipe;

@@ -176,8 +176,9 @@ struct StageBand {
 // is summed per lane, then across the group.  G holds the totals (particle count, cell
 // table length), C the particle's own instance; band is the particle's place in its
 // wavefront's LDS staging band
-// (unique in the workgroup), gbase its group's first lane in the wavefront.
-template <int L>
+// (unique in the workgroup), gbase its group's first lane in the wavefront.  FAR (L = 1): lists
+// beyond the int16 window too (kSeqList).
+template <int L, bool FAR = false>
 __device__ __forceinline__ void density_particle(const StepConsts& G, const StepConsts& C, int i, uint32_t l,
                                                  StageBand<L> band, uint32_t gbase, float4* pos, float4* vel,
                                                  const uint32_t* __restrict__ cs, float* __restrict__ rhoA,
@@ -189,9 +190,14 @@ __device__ __forceinline__ void density_particle(const StepConsts& G, const Step
     const size_t stride = (size_t)G.n;
     float acc = 0.0f;
     uint32_t cnt = 0;
-    // first and one past the last candidate: every list entry fits an int16 offset when the
+    // first and one past the last candidate: the neighbours lie in the list's window when the
     // candidates do (checked once per particle, not per hit)
     uint32_t klo = 0xffffffffu, khi = 0u;
+    // FAR: past the window the list is walked from one hit to the next (SeqWalk), so what has to
+    // stay below 2^16 is the distance of consecutive hits, bounded once per row with hits: from
+    // the first candidate of the last such row (kprev) to the end of this one
+    uint32_t kprev = 0u;
+    bool far = false;
     // L = 1 appends its hits in slot order: the next staged slot is reached from the last by a
     // step that alternates between 1 (the other half of the word) and the band's row pitch
     // less 1, in place of working out its address from the count on every hit
@@ -224,6 +230,7 @@ __device__ __forceinline__ void density_particle(const StepConsts& G, const Step
         klo = min(klo, k0);
         khi = max(khi, k1);
         if constexpr (L == 1) {
+            const uint32_t before = cnt;
             auto walk = [&](auto checked) {
                 uint32_t off = k0 * 16u;
                 const uint32_t end = k1 * 16u;
@@ -240,6 +247,10 @@ __device__ __forceinline__ void density_particle(const StepConsts& G, const Step
             // row's hits need no capacity checks (a wave-uniform choice)
             if (__ballot(cnt + (k1 - k0) > kCap) == 0) walk(std::false_type{});
             else walk(std::true_type{});
+            if (FAR && cnt != before) {
+                far |= k1 - (before ? kprev : klo) > 65536u;
+                kprev = k0;
+            }
         } else {
             for (uint32_t base = k0; base < k1; base += L) {
                 const uint32_t k = base + l;
@@ -271,8 +282,6 @@ __device__ __forceinline__ void density_particle(const StepConsts& G, const Step
     }
 #pragma unroll
     for (int o = 1; o < L; o <<= 1) acc += __shfl_xor(acc, o);
-    // the lanes of a group walk the same rows, so they agree on this
-    const bool wide = klo < khi && (klo + 32768u < (uint32_t)i || khi > (uint32_t)i + 32768u);
     const uint32_t staged = cnt < kCap ? cnt : kCap;
     // the staged slots as 32-bit words (two slots each), the group's lanes taking turns
     uint32_t* words = reinterpret_cast<uint32_t*>(nl);
@@ -280,15 +289,20 @@ __device__ __forceinline__ void density_particle(const StepConsts& G, const Step
         words[(size_t)(t >> 1) * stride + i] = band.word(t, staged);
     }
     if (l == 0) {
-        // a particle with a far neighbour is rescanned by the force pass, as one past the cap
-        nn[i] = wide && cnt <= (uint32_t)kListCap ? (uint32_t)kListCap + 1u : cnt;
+        // a particle past the cap, or with neighbours its list cannot reach, is rescanned by the
+        // force pass
+        const bool inside = klo >= khi || (klo + kListWindow >= (uint32_t)i && khi <= (uint32_t)i + kListWindow);
+        uint32_t head = cnt;
+        if (cnt > (uint32_t)kListCap) head = kNoList;
+        else if (!inside) head = FAR && !far && (uint32_t)i - klo < kSeqMaxBack ? seq_head(cnt, (uint32_t)i - klo) : kNoList;
+        nn[i] = head;
         store_density(C, i, acc, pos, vel, rhoA);
     }
 }
 
 // Plain step: L lanes per particle (1, 2, 4, 8, 16, 32 or 64), particle gt / L.  Groups are aligned,
 // so a whole group leaves together at the end of the range.
-template <int L>
+template <int L, bool FAR = false>
 __global__ __launch_bounds__(kDensityThreads) void naive_density_kernel(StepConsts G, float4* pos, float4* vel,
                                                                          const uint32_t* __restrict__ cs,
                                                                          float* __restrict__ rhoA,
@@ -301,7 +315,7 @@ __global__ __launch_bounds__(kDensityThreads) void naive_density_kernel(StepCons
     if (i >= G.n) return;
     const uint32_t lane = threadIdx.x & 63u;
     const StageBand<L> band{s_stage[threadIdx.x >> 6], lane / L};
-    density_particle<L>(G, G, i, gt & (L - 1), band, lane & ~(uint32_t)(L - 1), pos, vel, cs, rhoA, nl, nn);
+    density_particle<L, FAR>(G, G, i, gt & (L - 1), band, lane & ~(uint32_t)(L - 1), pos, vel, cs, rhoA, nl, nn);
 }
 
 // Batched form: each instance has its own lanes per particle and its own thread range, which
@@ -766,6 +780,12 @@ inline int blocks_for(int64_t n, int t) { return (int)((n + t - 1) / t); }
 
 constexpr int kDiagBlocks = 512;
 
+// Above this many particles the one-lane density pass writes lists beyond the int16 window.
+// Its bookkeeping costs 1% of the step on 1,048,576 particles in 128 layers of cells, where no
+// particle needs it (0.2112 against 0.2092 ms per step); on 4.2M in as many layers every
+// particle does (1.36 against 1.92 ms per step).
+constexpr int64_t kFarParticles = int64_t(1) << 20;
+
 hipError_t launch_fill_u32(uint32_t* p, uint32_t v, int64_t n, hipStream_t s) {
     if (n > 0) fill_u32_kernel<<<blocks_for(n, 256), 256, 0, s>>>(p, v, n);
     return hipGetLastError();
@@ -803,11 +823,11 @@ hipError_t launch_rekey(sph_ctx* c, hipStream_t s) {
     return hipGetLastError();
 }
 
-template <int L>
+template <int L, bool FAR = false>
 void launch_density_lanes(sph_ctx* c, hipStream_t s) {
     const int bs = c->density_block;
     const Buffers& b = c->b;
-    naive_density_kernel<L><<<blocks_for(c->n * L, bs), bs, 0, s>>>(c->sc, b.posA, b.velA, b.cs, b.rhoA, b.nl, b.nn);
+    naive_density_kernel<L, FAR><<<blocks_for(c->n * L, bs), bs, 0, s>>>(c->sc, b.posA, b.velA, b.cs, b.rhoA, b.nl, b.nn);
 }
 
 hipError_t launch_density(sph_ctx* c, hipStream_t s) {
@@ -832,7 +852,10 @@ hipError_t launch_density(sph_ctx* c, hipStream_t s) {
         case 16: launch_density_lanes<16>(c, s); break;
         case 32: launch_density_lanes<32>(c, s); break;
         case 64: launch_density_lanes<64>(c, s); break;
-        default: launch_density_lanes<1>(c, s); break;
+        default:
+            if (c->n > kFarParticles) launch_density_lanes<1, true>(c, s);
+            else launch_density_lanes<1>(c, s);
+            break;
     }
     return hipGetLastError();
 }
