@@ -80,7 +80,7 @@ __device__ __forceinline__ void walk_neighbours(const StepConsts& C, int i, floa
     }
 }
 
-// The same walk with L lanes per particle: lane l visits list slots l, l + L, ... (or every
+// The same walk with L lanes per particle: lane l visits list slots l, l + L, ... (and every
 // L-th candidate of each row past the list); the caller adds the lanes' sums.
 template <int L, typename F>
 __device__ __forceinline__ void walk_neighbours_lanes(const StepConsts& C, int i, uint32_t l, float4 p,
@@ -90,18 +90,23 @@ __device__ __forceinline__ void walk_neighbours_lanes(const StepConsts& C, int i
     if constexpr (L == 1) {
         walk_neighbours(C, i, p, pos, cs, nl, nn, f);
     } else {
-        const uint32_t cnt = nn[i];
-        if (cnt <= (uint32_t)kListCap) {
-            for (uint32_t t = l; t < cnt; t += L) f(list_decode(nl[list_at(C.n, i, t)], i));
-        } else {
+        const uint32_t head = nn[i];
+        const uint32_t cnt = head < kNoList ? min(head, (uint32_t)kListCap) : 0u;
+        for (uint32_t t = l; t < cnt; t += L) f(list_decode(nl[list_at(C.n, i, t)], i));
+        if (head > (uint32_t)kListCap) {
             const __amdgpu_buffer_rsrc_t rcs = make_rsrc(cs, ((uint32_t)C.cell_off + (uint32_t)C.n_cells + 1u) * 4u);
+            ListTail tail;
+            if (head < kNoList) {
+                const uint32_t last = list_decode(nl[list_at(C.n, i, kListCap - 1)], i);
+                tail = ListTail(last, pos[last], C);
+            }
             for_each_row_range<L>(p.x, p.y, p.z, C, rcs, l, [&](uint32_t k0, uint32_t k1) {
                 for (uint32_t k = k0 + l; k < k1; k += L) {
                     const float4 q = pos[k];
                     const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
                     if (dx * dx + dy * dy + dz * dz <= C.h2) f(k);
                 }
-            });
+            }, tail);
         }
     }
 }

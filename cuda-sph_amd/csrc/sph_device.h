@@ -2,6 +2,7 @@
 // reverse-mode kernels (sph_adjoint.hip).  The adjoint recomputes the force pass with the
 // same code as the step, so its recomputed forward is bitwise the step's own.
 #pragma once
+#include <limits.h>
 #include <math.h>
 
 #include "sph_internal.h"
@@ -286,21 +287,43 @@ __device__ __forceinline__ void for_each_row(float px, float py, float pz, const
     }
 }
 
+// Where the scan of a particle's candidates starts: at the first candidate k in the row of cells
+// (cy, cz), or, without a list, at its first row (cy = cz = INT_MIN stands for it).
+struct ListTail {
+    uint32_t k = 0u;
+    int cy = INT_MIN, cz = INT_MIN;
+    ListTail() = default;
+    // after its last listed neighbour, in the row that holds it (grid_coord gives the cell that
+    // it was sorted by)
+    __device__ __forceinline__ ListTail(uint32_t last, float4 q, const StepConsts& C)
+        : k(last + 1u), cy(grid_coord(q.y, 1, C)), cz(grid_coord(q.z, 2, C)) {}
+};
+
+template <typename F>
+__device__ __forceinline__ void for_each_candidate(float px, float py, float pz, const StepConsts& C,
+                                                   const uint32_t* __restrict__ cs, F&& f) {
+    for_each_row(px, py, pz, C, [&](int c) { return cs[c]; }, [&](uint32_t k0, uint32_t k1) {
+        for (uint32_t k = k0; k < k1; ++k) f(k);
+    });
+}
+
 // for_each_row for a group of L lanes sharing one particle (groups aligned in the
 // wavefront, l the lane's index in its group): the particle's (cy, cz) pairs are numbered
 // t = 0, 1, ... in for_each_row's order, lane l works out the rows of pairs l, l + L, ...
 // (geometry and cell-table entries), and every lane of the group then gets f(k0, k1) for
 // each row in order, the row's candidate range taken from the lane that owns it.  Rows the
 // sphere misses are skipped; rows without candidates are passed on (k0 == k1).
+// From the tail's start on, without the candidates before the tail's first.
 template <int L, typename F>
 __device__ __forceinline__ void for_each_row_range(float px, float py, float pz, const StepConsts& C,
-                                                   __amdgpu_buffer_rsrc_t rcs, uint32_t l, F&& f) {
+                                                   __amdgpu_buffer_rsrc_t rcs, uint32_t l, F&& f,
+                                                   ListTail tail = ListTail()) {
     const int gbase = (int)((threadIdx.x & 63u) & ~(uint32_t)(L - 1));
     const RowGrid R(px, py, pz, C);
     const int ny = R.yhi - R.ylo + 1;
     const int npairs = ny * (R.zhi - R.zlo + 1);
     const float inv_ny = 1.0f / (float)ny;
-    for (int t0 = 0; t0 < npairs; t0 += L) {
+    for (int t0 = ny * (max(tail.cz, R.zlo) - R.zlo) + max(tail.cy, R.ylo) - R.ylo; t0 < npairs; t0 += L) {
         uint32_t a0 = 0xffffffffu, a1 = 0u;  // an empty range unless the row exists
         const int t = t0 + (int)l;
         if (t < npairs) {
@@ -310,6 +333,7 @@ __device__ __forceinline__ void for_each_row_range(float px, float py, float pz,
             uint32_t q0, q1;
             if (R.row(cy, R.rest_z(cz, C), C, q0, q1))
                 RowGrid::range(row0, q0, q1, C, [&](int c) { return ld_u32(rcs, (uint32_t)c * 4u); }, a0, a1);
+            a0 = max(a0, tail.k);
         }
         const int last = min(L, npairs - t0);
         for (int j = 0; j < last; ++j) {
@@ -317,14 +341,6 @@ __device__ __forceinline__ void for_each_row_range(float px, float py, float pz,
             if (k0 <= k1) f(k0, k1);
         }
     }
-}
-
-template <typename F>
-__device__ __forceinline__ void for_each_candidate(float px, float py, float pz, const StepConsts& C,
-                                                   const uint32_t* __restrict__ cs, F&& f) {
-    for_each_row(px, py, pz, C, [&](int c) { return cs[c]; }, [&](uint32_t k0, uint32_t k1) {
-        for (uint32_t k = k0; k < k1; ++k) f(k);
-    });
 }
 
 // ---------------------------------------------------------------------------------------
@@ -515,6 +531,11 @@ __device__ __forceinline__ uint32_t finish_particle(const StepConsts& C, int i, 
 //                 next, so a walk from the first candidate on restores them (SeqWalk).  A 4.2M
 //                 particle dam break, whose layers of cells hold 33,000 particles each, left
 //                 its particles to a rescan without this: force 1,115 us per launch.
+//   <= kTailCount the count, more than there are slots: the first kListCap neighbours are listed,
+//                 within the window; the others are among the candidates after the last of
+//                 them, in its row of cells and the rows after it (ListTail).  A reader with one
+//                 lane per particle scans all candidates instead: the walk's second loop costs
+//                 the force pass registers it cannot spare (1M dam break, 59 -> 62 us).
 //   else          no list: the particle's candidates are scanned again, by a reader with several
 //                 lanes per particle also in place of a kSeqList walk.
 constexpr uint32_t kSeqList = 0x80000000u;
@@ -522,6 +543,11 @@ constexpr uint32_t kNoList = 0x7fffffffu;
 constexpr int kSeqCountBits = 10;
 constexpr uint32_t kSeqMaxBack = 1u << (31 - kSeqCountBits);
 constexpr uint32_t kListWindow = 1u << 15;
+// Past twice the slots most candidates lie after the list: one scan of all is cheaper then (the
+// dense instances of the 64-box batch, 2,000 neighbours: force 1,082 us against 1,162 with their
+// lists walked first; the 16,384-particle box, 102 neighbours, at 32 lanes: force 15.0 us with the
+// list against 19.6, pullback 26.8 against 32.4).
+constexpr uint32_t kTailCount = 2u * (uint32_t)kListCap;
 static_assert(kListCap < (1 << kSeqCountBits), "the count fits its field");
 __device__ __forceinline__ uint32_t seq_head(uint32_t cnt, uint32_t back) {
     return kSeqList | (back << kSeqCountBits) | cnt;
@@ -574,9 +600,6 @@ struct PairSums {
 #define SPH_FORCE_UNROLL 4
 #endif
 constexpr int kForceUnroll = SPH_FORCE_UNROLL;
-#ifndef SPH_FORCE_PREFETCH
-#define SPH_FORCE_PREFETCH 1
-#endif
 
 // Pressure and viscosity sums of particle i over its neighbour list (or, for a particle
 // with more neighbours than list slots, a rescan of its candidates).  The list holds the
@@ -650,7 +673,7 @@ __device__ __forceinline__ PairSums naive_pair_sums(const StepConsts& C, int i, 
 }
 
 // The same sums with L lanes per particle (L = 1 is naive_pair_sums): lane l of the group
-// walks list slots l, l + L, ... (or, past the list, every L-th candidate of each row), and
+// walks list slots l, l + L, ... (and, past the list, every L-th candidate of each row), and
 // the partial sums are added across the group; every lane of the group returns the total.
 template <int L>
 __device__ __forceinline__ PairSums naive_pair_sums_lanes(const StepConsts& C, int i, uint32_t l, int n, float4 p,
@@ -665,31 +688,29 @@ __device__ __forceinline__ PairSums naive_pair_sums_lanes(const StepConsts& C, i
         const __amdgpu_buffer_rsrc_t rpos = make_rsrc(pos, (uint32_t)n * 16u);
         const __amdgpu_buffer_rsrc_t rvel = make_rsrc(vel, (uint32_t)n * 16u);
         PairSums S;
-        const uint32_t cnt = nn[i];
-        if (cnt <= (uint32_t)kListCap) {
-#if SPH_FORCE_PREFETCH
-            // the lane's next list slot is loaded while this slot's neighbour is gathered
-            uint32_t kn = l < cnt ? list_decode(nl[list_at(n, i, l)], i) : 0u;
-            for (uint32_t t = l; t < cnt; t += L) {
-                const uint32_t k = kn;
-                if (t + L < cnt) kn = list_decode(nl[list_at(n, i, t + L)], i);
-                S.add(C, p, v, ld_f4(rpos, k * 16u), ld_f4(rvel, k * 16u), k == (uint32_t)i);
-            }
-#else
-            for (uint32_t t = l; t < cnt; t += L) {
-                const uint32_t k = list_decode(nl[list_at(n, i, t)], i);
-                S.add(C, p, v, ld_f4(rpos, k * 16u), ld_f4(rvel, k * 16u), k == (uint32_t)i);
-            }
-#endif
-        } else {
+        const uint32_t head = nn[i];
+        const uint32_t cnt = head < kNoList ? min(head, (uint32_t)kListCap) : 0u;
+        // the lane's next list slot is loaded while this slot's neighbour is gathered
+        uint32_t kn = l < cnt ? list_decode(nl[list_at(n, i, l)], i) : 0u;
+        for (uint32_t t = l; t < cnt; t += L) {
+            const uint32_t k = kn;
+            if (t + L < cnt) kn = list_decode(nl[list_at(n, i, t + L)], i);
+            S.add(C, p, v, ld_f4(rpos, k * 16u), ld_f4(rvel, k * 16u), k == (uint32_t)i);
+        }
+        if (head > (uint32_t)kListCap) {
             const __amdgpu_buffer_rsrc_t rcs = make_rsrc(cs, ((uint32_t)C.cell_off + (uint32_t)C.n_cells + 1u) * 4u);
+            ListTail tail;
+            if (head < kNoList) {
+                const uint32_t last = list_decode(nl[list_at(n, i, kListCap - 1)], i);
+                tail = ListTail(last, ld_f4(rpos, last * 16u), C);
+            }
             for_each_row_range<L>(p.x, p.y, p.z, C, rcs, l, [&](uint32_t k0, uint32_t k1) {
                 for (uint32_t k = k0 + l; k < k1; k += L) {
                     const float4 q = ld_f4(rpos, k * 16u);
                     const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
                     if (dx * dx + dy * dy + dz * dz <= C.h2 && k != (uint32_t)i) S.add(C, p, v, q, ld_f4(rvel, k * 16u));
                 }
-            });
+            }, tail);
         }
 #pragma unroll
         for (int o = 1; o < L; o <<= 1) {

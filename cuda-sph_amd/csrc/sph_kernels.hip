@@ -289,12 +289,14 @@ __device__ __forceinline__ void density_particle(const StepConsts& G, const Step
         words[(size_t)(t >> 1) * stride + i] = band.word(t, staged);
     }
     if (l == 0) {
-        // a particle past the cap, or with neighbours its list cannot reach, is rescanned by the
-        // force pass
+        // past the cap the list holds the first neighbours; a particle with neighbours its list
+        // cannot reach is rescanned by the force pass
         const bool inside = klo >= khi || (klo + kListWindow >= (uint32_t)i && khi <= (uint32_t)i + kListWindow);
-        uint32_t head = cnt;
-        if (cnt > (uint32_t)kListCap) head = kNoList;
-        else if (!inside) head = FAR && !far && (uint32_t)i - klo < kSeqMaxBack ? seq_head(cnt, (uint32_t)i - klo) : kNoList;
+        uint32_t head = cnt <= kTailCount ? cnt : kNoList;
+        if (!inside) {
+            const bool seq = FAR && cnt <= (uint32_t)kListCap && !far && (uint32_t)i - klo < kSeqMaxBack;
+            head = seq ? seq_head(cnt, (uint32_t)i - klo) : kNoList;
+        }
         nn[i] = head;
         store_density(C, i, acc, pos, vel, rhoA);
     }

@@ -73,3 +73,23 @@ def test_pullback_from_far_lists(gpu):
         got.append([t.double() for t in ctx.adjoint_read()])
     for a, b in zip(*got):
         assert float((a - b).norm() / b.norm()) <= TOL
+
+
+# 96 list slots; up to 192 neighbours the force pass walks the list and then the candidates after
+# its last neighbour, past that it scans all candidates.  h sets the mean: 60, 97, 150 and 250.
+@pytest.mark.parametrize("lanes", [1, 2, 8, 64])
+@pytest.mark.parametrize("mean", [60, 97, 150, 250])
+def test_lists_past_their_slots(gpu, mean, lanes):
+    n = 3001
+    h = (mean / (n / 0.4 ** 3) / (4.0 / 3.0 * np.pi)) ** (1.0 / 3.0)
+    w = box_uniform(n, seed=73, h=h)
+    rng = np.random.default_rng(74)
+    pos = w.state.position.astype(np.float32).astype(np.float64)
+    vel = rng.normal(0.0, 0.3, size=(n, 3)).astype(np.float32).astype(np.float64)
+    strat = NaiveSPHStrategy(w.params, constants=w.constants, device=gpu, lanes=lanes)
+    out = strat.compute_next_state(SimulationState(pos, vel, np.zeros(n)))
+    rp, rv, rrho, _, _ = oracle.step(pos, vel, consts=w.constants, ext=w.params.external_force, dt=1e-3,
+                                     space=w.params.space_size, voxel=w.params.voxel_size)
+    assert (np.abs(out.density - rrho) / rrho).max() <= TOL
+    assert (np.abs(out.position - rp) / np.maximum(np.abs(rp), 1e-3)).max() <= TOL
+    assert np.abs(out.velocity - rv).max() / np.abs(rv).max() <= TOL
