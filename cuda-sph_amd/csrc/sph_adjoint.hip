@@ -100,13 +100,13 @@ __device__ __forceinline__ void walk_neighbours_lanes(const StepConsts& C, int i
                 const uint32_t last = list_decode(nl[list_at(C.n, i, kListCap - 1)], i);
                 tail = ListTail(last, pos[last], C);
             }
-            for_each_row_range<L>(p.x, p.y, p.z, C, rcs, l, [&](uint32_t k0, uint32_t k1) {
-                for (uint32_t k = k0 + l; k < k1; k += L) {
-                    const float4 q = pos[k];
+            for_each_batch<L>(
+                p.x, p.y, p.z, C, rcs, make_rsrc(pos, (uint32_t)C.n * 16u), l, [](uint32_t, uint32_t) {},
+                [&](uint32_t k, float4 q, bool valid) {
                     const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
-                    if (dx * dx + dy * dy + dz * dz <= C.h2) f(k);
-                }
-            }, tail);
+                    if (valid && dx * dx + dy * dy + dz * dz <= C.h2) f(k);
+                },
+                tail);
         }
     }
 }

@@ -310,35 +310,60 @@ __device__ __forceinline__ void for_each_candidate(float px, float py, float pz,
 // for_each_row for a group of L lanes sharing one particle (groups aligned in the
 // wavefront, l the lane's index in its group): the particle's (cy, cz) pairs are numbered
 // t = 0, 1, ... in for_each_row's order, lane l works out the rows of pairs l, l + L, ...
-// (geometry and cell-table entries), and every lane of the group then gets f(k0, k1) for
-// each row in order, the row's candidate range taken from the lane that owns it.  Rows the
-// sphere misses are skipped; rows without candidates are passed on (k0 == k1).
-// From the tail's start on, without the candidates before the tail's first.
-template <int L, typename F>
-__device__ __forceinline__ void for_each_row_range(float px, float py, float pz, const StepConsts& C,
-                                                   __amdgpu_buffer_rsrc_t rcs, uint32_t l, F&& f,
-                                                   ListTail tail = ListTail()) {
+// (geometry and cell-table entries), and the group then takes the rows' candidates in order,
+// L at a time and a row's rest by itself: f(k, q, valid) is called by all lanes of the group
+// together, lane l with the candidate k = k0 + l + L m of the row and q = pos[k] (valid: k lies
+// in the row).  The next batch's positions are loaded before f gets this one's, so a group does
+// not wait for each batch in turn.  From the tail's start on, without the candidates before the
+// tail's first.  rows(k0, k1) gets the lane's own row ranges.
+template <int L, typename RowF, typename F>
+__device__ __forceinline__ void for_each_batch(float px, float py, float pz, const StepConsts& C,
+                                               __amdgpu_buffer_rsrc_t rcs, __amdgpu_buffer_rsrc_t rpos, uint32_t l,
+                                               RowF&& rows, F&& f, ListTail tail = ListTail()) {
     const int gbase = (int)((threadIdx.x & 63u) & ~(uint32_t)(L - 1));
     const RowGrid R(px, py, pz, C);
     const int ny = R.yhi - R.ylo + 1;
     const int npairs = ny * (R.zhi - R.zlo + 1);
     const float inv_ny = 1.0f / (float)ny;
+    constexpr uint64_t group = L == 64 ? ~0ull : (1ull << (L & 63)) - 1ull;
     for (int t0 = ny * (max(tail.cz, R.zlo) - R.zlo) + max(tail.cy, R.ylo) - R.ylo; t0 < npairs; t0 += L) {
-        uint32_t a0 = 0xffffffffu, a1 = 0u;  // an empty range unless the row exists
+        uint32_t a0 = 0u, a1 = 0u;
         const int t = t0 + (int)l;
         if (t < npairs) {
             const int q = (int)(((float)t + 0.5f) * inv_ny);  // exact: t and ny are small
             const int cz = R.zlo + q, cy = R.ylo + (t - q * ny);
             const int row0 = C.cell_off + C.dims[0] * (cy + C.dims[1] * cz);
             uint32_t q0, q1;
-            if (R.row(cy, R.rest_z(cz, C), C, q0, q1))
+            if (R.row(cy, R.rest_z(cz, C), C, q0, q1)) {
                 RowGrid::range(row0, q0, q1, C, [&](int c) { return ld_u32(rcs, (uint32_t)c * 4u); }, a0, a1);
-            a0 = max(a0, tail.k);
+                a0 = max(a0, tail.k);
+                if (a0 < a1) rows(a0, a1);
+            }
         }
-        const int last = min(L, npairs - t0);
-        for (int j = 0; j < last; ++j) {
-            const uint32_t k0 = __shfl(a0, gbase + j), k1 = __shfl(a1, gbase + j);
-            if (k0 <= k1) f(k0, k1);
+        uint64_t left = (__ballot(a0 < a1) >> gbase) & group;  // the rows that hold candidates
+        uint32_t b = 0u, e = 0u;
+        auto next_row = [&]() {
+            const int j = gbase + __ffsll((unsigned long long)left) - 1;
+            left &= left - 1ull;
+            b = __shfl(a0, j);
+            e = __shfl(a1, j);
+        };
+        if (left == 0ull) continue;
+        next_row();
+        float4 q = ld_f4(rpos, min(b + l, e - 1u) * 16u);
+        while (true) {
+            const uint32_t k = b + l;
+            const float4 qk = q;
+            const bool valid = k < e;
+            b += L;
+            bool more = true;
+            if (b >= e) {
+                more = left != 0ull;
+                if (more) next_row();
+            }
+            if (more) q = ld_f4(rpos, min(b + l, e - 1u) * 16u);
+            f(k, qk, valid);
+            if (!more) break;
         }
     }
 }
@@ -704,13 +729,14 @@ __device__ __forceinline__ PairSums naive_pair_sums_lanes(const StepConsts& C, i
                 const uint32_t last = list_decode(nl[list_at(n, i, kListCap - 1)], i);
                 tail = ListTail(last, ld_f4(rpos, last * 16u), C);
             }
-            for_each_row_range<L>(p.x, p.y, p.z, C, rcs, l, [&](uint32_t k0, uint32_t k1) {
-                for (uint32_t k = k0 + l; k < k1; k += L) {
-                    const float4 q = ld_f4(rpos, k * 16u);
+            for_each_batch<L>(
+                p.x, p.y, p.z, C, rcs, rpos, l, [](uint32_t, uint32_t) {},
+                [&](uint32_t k, float4 q, bool valid) {
                     const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
-                    if (dx * dx + dy * dy + dz * dz <= C.h2 && k != (uint32_t)i) S.add(C, p, v, q, ld_f4(rvel, k * 16u));
-                }
-            }, tail);
+                    if (valid && dx * dx + dy * dy + dz * dz <= C.h2 && k != (uint32_t)i)
+                        S.add(C, p, v, q, ld_f4(rvel, k * 16u));
+                },
+                tail);
         }
 #pragma unroll
         for (int o = 1; o < L; o <<= 1) {

@@ -225,11 +225,11 @@ __device__ __forceinline__ void density_particle(const StepConsts& G, const Step
             ++cnt;
         }
     };
-    // candidates k0 .. k1 - 1 of one row
-    auto run_row = [&](uint32_t k0, uint32_t k1) {
-        klo = min(klo, k0);
-        khi = max(khi, k1);
-        if constexpr (L == 1) {
+    if constexpr (L == 1) {
+        // candidates k0 .. k1 - 1 of one row
+        auto run_row = [&](uint32_t k0, uint32_t k1) {
+            klo = min(klo, k0);
+            khi = max(khi, k1);
             const uint32_t before = cnt;
             auto walk = [&](auto checked) {
                 uint32_t off = k0 * 16u;
@@ -251,11 +251,17 @@ __device__ __forceinline__ void density_particle(const StepConsts& G, const Step
                 far |= k1 - (before ? kprev : klo) > 65536u;
                 kprev = k0;
             }
-        } else {
-            for (uint32_t base = k0; base < k1; base += L) {
-                const uint32_t k = base + l;
-                const bool valid = k < k1;
-                const float4 q = ld_f4(rpos, (valid ? k : k0) * 16u);
+        };
+        for_each_row(p.x, p.y, p.z, C, [&](int c) { return ld_u32(rcs, (uint32_t)c * 4u); }, run_row);
+    } else {
+        // one candidate per lane of the group, hits ranked by a ballot
+        for_each_batch<L>(
+            p.x, p.y, p.z, C, rcs, rpos, l,
+            [&](uint32_t k0, uint32_t k1) {
+                klo = min(klo, k0);
+                khi = max(khi, k1);
+            },
+            [&](uint32_t k, float4 q, bool valid) {
                 const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
                 const float r2 = valid ? dx * dx + dy * dy + dz * dz : INFINITY;
                 const bool hit = r2 <= C.h2;
@@ -263,7 +269,7 @@ __device__ __forceinline__ void density_particle(const StepConsts& G, const Step
                     const float t = 1.0f - r2 * C.inv_h2;
                     acc += t * t * t;
                 }
-                constexpr uint64_t group = L == 64 ? ~0ull : (1ull << L) - 1ull;
+                constexpr uint64_t group = L == 64 ? ~0ull : (1ull << (L & 63)) - 1ull;
                 const uint64_t gm = (__ballot(hit) >> gbase) & group;
                 if (hit) {
                     const uint32_t slot = cnt + (uint32_t)__popcll(gm & ((1ull << l) - 1ull));
@@ -271,14 +277,12 @@ __device__ __forceinline__ void density_particle(const StepConsts& G, const Step
                     else if (slot < (uint32_t)kListCap) nl[list_at(G.n, i, slot)] = list_encode(k, i);
                 }
                 cnt += (uint32_t)__popcll(gm);
-            }
+            });
+#pragma unroll
+        for (int o = 1; o < L; o <<= 1) {
+            klo = min(klo, (uint32_t)__shfl_xor(klo, o));
+            khi = max(khi, (uint32_t)__shfl_xor(khi, o));
         }
-    };
-    if constexpr (L == 1) {
-        for_each_row(p.x, p.y, p.z, C, [&](int c) { return ld_u32(rcs, (uint32_t)c * 4u); }, run_row);
-    } else {
-        // the group shares the row walk; rows without candidates still bound klo, khi
-        for_each_row_range<L>(p.x, p.y, p.z, C, rcs, l, run_row);
     }
 #pragma unroll
     for (int o = 1; o < L; o <<= 1) acc += __shfl_xor(acc, o);
