@@ -75,7 +75,7 @@ __device__ __forceinline__ void walk_neighbours(const StepConsts& C, int i, floa
         for_each_candidate(p.x, p.y, p.z, C, cs, [&](uint32_t k) {
             const float4 q = pos[k];
             const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
-            if (dx * dx + dy * dy + dz * dz <= C.h2) f(k);
+            if (norm2(dx, dy, dz) <= C.h2) f(k);
         });
     }
 }
@@ -104,7 +104,7 @@ __device__ __forceinline__ void walk_neighbours_lanes(const StepConsts& C, int i
                 p.x, p.y, p.z, C, rcs, make_rsrc(pos, (uint32_t)C.n * 16u), l, [](uint32_t, uint32_t) {},
                 [&](uint32_t k, float4 q, bool valid) {
                     const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
-                    if (valid && dx * dx + dy * dy + dz * dz <= C.h2) f(k);
+                    if (valid && norm2(dx, dy, dz) <= C.h2) f(k);
                 },
                 tail);
         }
@@ -224,7 +224,7 @@ __global__ __launch_bounds__(kAdjThreads) void adjoint_pair_kernel(
         if (j == (uint32_t)k) return;
         const float4 q = pos[j], w = vel[j], fj = fb[j];
         const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
-        const float r2 = dx * dx + dy * dy + dz * dz;
+        const float r2 = norm2(dx, dy, dz);
         const float rinv = rsqrtf(r2);
         const float r = r2 * rinv;
         const float hr = h - r;
@@ -287,7 +287,7 @@ __global__ __launch_bounds__(kAdjThreads) void adjoint_density_kernel(
     walk_neighbours_lanes<L>(C, k, lane, p, pos, cs, nl, nn, [&](uint32_t j) {
         const float4 q = pos[j];
         const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
-        const float u = fmaxf(1.0f - (dx * dx + dy * dy + dz * dz) * C.inv_h2, 0.0f);
+        const float u = fmaxf(1.0f - (norm2(dx, dy, dz)) * C.inv_h2, 0.0f);
         const float c = (rk + rt[j]) * u * u;
         ax += c * dx;
         ay += c * dy;

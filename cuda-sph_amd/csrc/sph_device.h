@@ -544,6 +544,13 @@ __device__ __forceinline__ uint32_t finish_particle(const StepConsts& C, int i, 
     return hash_particle<SLOT_KEYS>(C, pp.x, pp.y, pp.z, pid, (uint32_t)i, keyI, valI, flags);
 }
 
+// |d|^2 with its roundings spelled out: the compiler fuses the plain sum of squares around
+// different products in different copies of a loop, and the neighbour relation must be the same
+// from both particles, the sums the same from every kernel that forms them.
+__device__ __forceinline__ float norm2(float dx, float dy, float dz) {
+    return __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
+}
+
 // Neighbour lists.  Slots t and t + 1 (t even) of particle i share the 32-bit word (t / 2) * n
 // + i, so a lane reads two slots per load and consecutive particles' words are contiguous.  A
 // slot holds the low 16 bits of the neighbour's cell-ordered index minus the particle's own;
@@ -606,7 +613,7 @@ struct PairSums {
     __device__ __forceinline__ void add(const StepConsts& C, float4 p, float4 v, float4 q, float4 vj,
                                         bool self = false) {
         const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
-        const float r2 = dx * dx + dy * dy + dz * dz;
+        const float r2 = norm2(dx, dy, dz);
         const float rinv = self ? 0.0f : __builtin_amdgcn_rsqf(r2);
         const float hr = C.h - r2 * rinv;
         const float cp = (p.w + q.w) * vj.w * hr * hr * rinv;
@@ -691,7 +698,7 @@ __device__ __forceinline__ PairSums naive_pair_sums(const StepConsts& C, int i, 
         for_each_candidate(p.x, p.y, p.z, C, cs, [&](uint32_t k) {
             const float4 q = pos[k];
             const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
-            if (dx * dx + dy * dy + dz * dz <= C.h2 && k != (uint32_t)i) S.add(C, p, v, q, vel[k]);
+            if (norm2(dx, dy, dz) <= C.h2 && k != (uint32_t)i) S.add(C, p, v, q, vel[k]);
         });
     }
     return S;
@@ -733,7 +740,7 @@ __device__ __forceinline__ PairSums naive_pair_sums_lanes(const StepConsts& C, i
                 p.x, p.y, p.z, C, rcs, rpos, l, [](uint32_t, uint32_t) {},
                 [&](uint32_t k, float4 q, bool valid) {
                     const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
-                    if (valid && dx * dx + dy * dy + dz * dz <= C.h2 && k != (uint32_t)i)
+                    if (valid && norm2(dx, dy, dz) <= C.h2 && k != (uint32_t)i)
                         S.add(C, p, v, q, ld_f4(rvel, k * 16u));
                 },
                 tail);
@@ -749,6 +756,90 @@ __device__ __forceinline__ PairSums naive_pair_sums_lanes(const StepConsts& C, i
         }
         return S;
     }
+}
+
+// The sums of naive_pair_sums, to the same bits, by a group of L >= 8 lanes: the lanes work out the
+// terms of L pairs, keep them in LDS, and lanes 0 .. 5 each add one component of them up in the
+// list's (or the scan's) order.  buf: the group's kOrderedPairWords<L> words of LDS: per pair
+// the two coefficients and the components they multiply, kept apart by an odd pitch so that
+// the six lanes read six banks.
+template <int L>
+constexpr uint32_t kOrderedPitch = (uint32_t)L + 1u;
+template <int L>
+constexpr uint32_t kOrderedPairWords = 8u * kOrderedPitch<L>;
+template <int L>
+__device__ __forceinline__ PairSums naive_pair_sums_ordered(const StepConsts& C, int i, uint32_t l, int n, float4 p,
+                                                            float4 v, const float4* __restrict__ pos,
+                                                            const float4* __restrict__ vel,
+                                                            const uint32_t* __restrict__ cs,
+                                                            const ListEntry* __restrict__ nl,
+                                                            const uint32_t* __restrict__ nn, float* buf) {
+    static_assert(L >= 8, "six lanes add");
+    const __amdgpu_buffer_rsrc_t rpos = make_rsrc(pos, (uint32_t)n * 16u);
+    const __amdgpu_buffer_rsrc_t rvel = make_rsrc(vel, (uint32_t)n * 16u);
+    constexpr uint32_t kPitch = kOrderedPitch<L>;
+    const int gbase = (int)((threadIdx.x & 63u) & ~(uint32_t)(L - 1));
+    const uint32_t comp = l < 6u ? l : 5u;
+    const float* const coef = buf + (comp < 3u ? 0u : kPitch);
+    const float* const part = buf + (2u + comp) * kPitch;
+    float acc = 0.0f;
+    // the terms of one pair (PairSums::add) into place `at`
+    auto keep = [&](float4 q, float4 vj, bool self, uint32_t at) {
+        const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
+        const float r2 = norm2(dx, dy, dz);
+        const float rinv = self ? 0.0f : __builtin_amdgcn_rsqf(r2);
+        const float hr = C.h - r2 * rinv;
+        buf[at] = (p.w + q.w) * vj.w * hr * hr * rinv;
+        buf[kPitch + at] = hr * vj.w;
+        buf[2u * kPitch + at] = dx;
+        buf[3u * kPitch + at] = dy;
+        buf[4u * kPitch + at] = dz;
+        buf[5u * kPitch + at] = vj.x - v.x;
+        buf[6u * kPitch + at] = vj.y - v.y;
+        buf[7u * kPitch + at] = vj.z - v.z;
+    };
+    auto add = [&](uint32_t count) {
+        __builtin_amdgcn_wave_barrier();
+        for (uint32_t t = 0; t < count; ++t) acc += coef[t] * part[t];
+        __builtin_amdgcn_wave_barrier();
+    };
+    const uint32_t head = nn[i];
+    const uint32_t cnt = head < kNoList ? min(head, (uint32_t)kListCap) : 0u;
+    uint32_t kn = l < cnt ? list_decode(nl[list_at(n, i, l)], i) : (uint32_t)i;
+    for (uint32_t t = 0; t < cnt; t += L) {
+        const uint32_t k = kn;
+        const float4 q = ld_f4(rpos, k * 16u), w = ld_f4(rvel, k * 16u);
+        if (t + L + l < cnt) kn = list_decode(nl[list_at(n, i, t + L + l)], i);
+        keep(q, w, k == (uint32_t)i, l);
+        add(min((uint32_t)L, cnt - t));
+    }
+    if (head > (uint32_t)kListCap) {
+        const __amdgpu_buffer_rsrc_t rcs = make_rsrc(cs, ((uint32_t)C.cell_off + (uint32_t)C.n_cells + 1u) * 4u);
+        constexpr uint64_t group = L == 64 ? ~0ull : (1ull << (L & 63)) - 1ull;
+        ListTail tail;
+        if (head < kNoList) {
+            const uint32_t last = list_decode(nl[list_at(n, i, kListCap - 1)], i);
+            tail = ListTail(last, ld_f4(rpos, last * 16u), C);
+        }
+        for_each_batch<L>(
+            p.x, p.y, p.z, C, rcs, rpos, l, [](uint32_t, uint32_t) {},
+            [&](uint32_t k, float4 q, bool valid) {
+                const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
+                const bool hit = valid && norm2(dx, dy, dz) <= C.h2 && k != (uint32_t)i;
+                const uint64_t gm = (__ballot(hit) >> gbase) & group;
+                if (hit) keep(q, ld_f4(rvel, k * 16u), false, (uint32_t)__popcll(gm & ((1ull << l) - 1ull)));
+                add((uint32_t)__popcll(gm));
+            },
+            tail);
+    }
+    PairSums S;
+    S.ax = __shfl(acc, gbase);
+    S.ay = __shfl(acc, gbase + 1);
+    S.az = __shfl(acc, gbase + 2);
+    S.bx = __shfl(acc, gbase + 3);
+    S.by = __shfl(acc, gbase + 4);
+    S.bz = __shfl(acc, gbase + 5);
+    return S;
 }
 
 }  // namespace

@@ -234,6 +234,8 @@ bool cell_sort_global(const sph_ctx* c);
 // whether the force pass can count the keys it writes for the next step's counting sort:
 // a plain (not batched) NAIVE step on the global sort path
 bool count_in_force(const sph_ctx* c);
+// lanes that share a particle of a plain context with one lane per particle (ordered sums)
+int ordered_lanes(const sph_ctx* c);
 // whether such a force pass also adds the keys into the scan's tile sums (one lane per
 // particle)
 bool tile_sums_in_force(const sph_ctx* c);

@@ -167,6 +167,10 @@ struct StageBand {
     }
 };
 
+// ORDERED: hit terms of a particle kept in LDS between two additions (a multiple of 4, the last 4
+// for the zeros that fill the last float4)
+constexpr uint32_t kOrderedTerms = 128;
+
 // Density of cell-ordered particle i with L lanes per particle.  L = 1: the lane walks every
 // candidate row, two candidates in flight through 32-bit buffer offsets.  L = 2..16: a group
 // of L consecutive lanes of one wavefront shares the particle, walks the same rows and takes
@@ -177,12 +181,15 @@ struct StageBand {
 // table length), C the particle's own instance; band is the particle's place in its
 // wavefront's LDS staging band
 // (unique in the workgroup), gbase its group's first lane in the wavefront.  FAR (L = 1): lists
-// beyond the int16 window too (kSeqList).
-template <int L, bool FAR = false>
+// beyond the int16 window too (kSeqList).  ORDERED (L > 1): the density is summed over the hits
+// in list order, as one lane sums it, to the same bits: the group keeps the hits' terms in terms
+// (kOrderedTerms words of LDS) and adds them up from there.
+template <int L, bool FAR = false, bool ORDERED = false>
 __device__ __forceinline__ void density_particle(const StepConsts& G, const StepConsts& C, int i, uint32_t l,
                                                  StageBand<L> band, uint32_t gbase, float4* pos, float4* vel,
                                                  const uint32_t* __restrict__ cs, float* __restrict__ rhoA,
-                                                 ListEntry* __restrict__ nl, uint32_t* __restrict__ nn) {
+                                                 ListEntry* __restrict__ nl, uint32_t* __restrict__ nn,
+                                                 float* terms = nullptr) {
     constexpr uint32_t kCap = stage_cap<L>();
     const __amdgpu_buffer_rsrc_t rpos = make_rsrc(pos, (uint32_t)G.n * 16u);
     const __amdgpu_buffer_rsrc_t rcs = make_rsrc(cs, ((uint32_t)G.cs_cells + 1u) * 4u);
@@ -212,7 +219,7 @@ __device__ __forceinline__ void density_particle(const StepConsts& G, const Step
     // list; CHECKED: the list may be full (staged slots, then HBM slots, then only counted)
     auto visit = [&](float4 q, uint32_t k, auto checked) {
         const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
-        const float r2 = dx * dx + dy * dy + dz * dz;
+        const float r2 = norm2(dx, dy, dz);
         if (r2 <= C.h2) {
             const float t = 1.0f - r2 * C.inv_h2;
             acc += t * t * t;
@@ -254,6 +261,19 @@ __device__ __forceinline__ void density_particle(const StepConsts& G, const Step
         };
         for_each_row(p.x, p.y, p.z, C, [&](int c) { return ld_u32(rcs, (uint32_t)c * 4u); }, run_row);
     } else {
+        uint32_t kept = 0;  // terms not added yet
+        auto add_terms = [&]() {
+            // whole float4s: a term of zero adds nothing
+            if (l < 3u) terms[kept + l] = 0.0f;
+            for (uint32_t t = 0; t < kept; t += 4u) {
+                const float4 u = *reinterpret_cast<const float4*>(terms + t);
+                acc += u.x * u.x * u.x;
+                acc += u.y * u.y * u.y;
+                acc += u.z * u.z * u.z;
+                acc += u.w * u.w * u.w;
+            }
+            kept = 0;
+        };
         // one candidate per lane of the group, hits ranked by a ballot
         for_each_batch<L>(
             p.x, p.y, p.z, C, rcs, rpos, l,
@@ -263,29 +283,34 @@ __device__ __forceinline__ void density_particle(const StepConsts& G, const Step
             },
             [&](uint32_t k, float4 q, bool valid) {
                 const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
-                const float r2 = valid ? dx * dx + dy * dy + dz * dz : INFINITY;
+                const float r2 = valid ? norm2(dx, dy, dz) : INFINITY;
                 const bool hit = r2 <= C.h2;
-                if (hit) {
-                    const float t = 1.0f - r2 * C.inv_h2;
-                    acc += t * t * t;
-                }
+                const float t = 1.0f - r2 * C.inv_h2;
+                if (!ORDERED && hit) acc += t * t * t;
                 constexpr uint64_t group = L == 64 ? ~0ull : (1ull << (L & 63)) - 1ull;
                 const uint64_t gm = (__ballot(hit) >> gbase) & group;
+                if (ORDERED && kept + L > kOrderedTerms - 4u) add_terms();
                 if (hit) {
-                    const uint32_t slot = cnt + (uint32_t)__popcll(gm & ((1ull << l) - 1ull));
+                    const uint32_t before = (uint32_t)__popcll(gm & ((1ull << l) - 1ull));
+                    const uint32_t slot = cnt + before;
+                    if (ORDERED) terms[kept + before] = t;
                     if (slot < kCap) band.at(slot) = list_encode(k, i);
                     else if (slot < (uint32_t)kListCap) nl[list_at(G.n, i, slot)] = list_encode(k, i);
                 }
                 cnt += (uint32_t)__popcll(gm);
+                kept += (uint32_t)__popcll(gm);
             });
+        if (ORDERED) add_terms();
 #pragma unroll
         for (int o = 1; o < L; o <<= 1) {
             klo = min(klo, (uint32_t)__shfl_xor(klo, o));
             khi = max(khi, (uint32_t)__shfl_xor(khi, o));
         }
     }
+    if (!ORDERED) {
 #pragma unroll
-    for (int o = 1; o < L; o <<= 1) acc += __shfl_xor(acc, o);
+        for (int o = 1; o < L; o <<= 1) acc += __shfl_xor(acc, o);
+    }
     const uint32_t staged = cnt < kCap ? cnt : kCap;
     // the staged slots as 32-bit words (two slots each), the group's lanes taking turns
     uint32_t* words = reinterpret_cast<uint32_t*>(nl);
@@ -308,7 +333,7 @@ __device__ __forceinline__ void density_particle(const StepConsts& G, const Step
 
 // Plain step: L lanes per particle (1, 2, 4, 8, 16, 32 or 64), particle gt / L.  Groups are aligned,
 // so a whole group leaves together at the end of the range.
-template <int L, bool FAR = false>
+template <int L, bool FAR = false, bool ORDERED = false>
 __global__ __launch_bounds__(kDensityThreads) void naive_density_kernel(StepConsts G, float4* pos, float4* vel,
                                                                          const uint32_t* __restrict__ cs,
                                                                          float* __restrict__ rhoA,
@@ -321,7 +346,9 @@ __global__ __launch_bounds__(kDensityThreads) void naive_density_kernel(StepCons
     if (i >= G.n) return;
     const uint32_t lane = threadIdx.x & 63u;
     const StageBand<L> band{s_stage[threadIdx.x >> 6], lane / L};
-    density_particle<L, FAR>(G, G, i, gt & (L - 1), band, lane & ~(uint32_t)(L - 1), pos, vel, cs, rhoA, nl, nn);
+    __shared__ __align__(16) float s_terms[ORDERED ? kDensityThreads / L : 1][ORDERED ? kOrderedTerms : 1];
+    density_particle<L, FAR, ORDERED>(G, G, i, gt & (L - 1), band, lane & ~(uint32_t)(L - 1), pos, vel, cs, rhoA, nl, nn,
+                                      s_terms[ORDERED ? threadIdx.x / L : 0]);
 }
 
 // Batched form: each instance has its own lanes per particle and its own thread range, which
@@ -384,7 +411,7 @@ __global__ __launch_bounds__(kDensityThreads) void naive_density_batch_kernel(St
 // their gathers in flight); a particle with more neighbours than list slots rescans its
 // candidates instead.  With L lanes per particle the group splits the list (or the rescan)
 // and lane 0 finishes the particle.  MODE selects the wall collision at compile time.
-template <int MODE, int L = 1, bool COUNT = false>
+template <int MODE, int L = 1, bool COUNT = false, bool ORDERED = false>
 __global__ __launch_bounds__(256) void naive_force_kernel(
     StepConsts G, const float4* __restrict__ pos, const float4* __restrict__ vel, const uint32_t* __restrict__ pidA,
     const float* __restrict__ rhoA, const uint32_t* __restrict__ cs, const ListEntry* __restrict__ nl,
@@ -399,7 +426,13 @@ __global__ __launch_bounds__(256) void naive_force_kernel(
     if (i >= G.n) return;
     const StepConsts& C = G;
     const float4 p = pos[i], v = vel[i];
-    const PairSums S = naive_pair_sums_lanes<L>(C, i, gt & (L - 1), G.n, p, v, pos, vel, cs, nl, nn);
+    PairSums S;
+    if constexpr (ORDERED) {
+        __shared__ float s_pairs[256 / L][kOrderedPairWords<L>];
+        S = naive_pair_sums_ordered<L>(C, i, gt & (L - 1), G.n, p, v, pos, vel, cs, nl, nn, s_pairs[threadIdx.x / L]);
+    } else {
+        S = naive_pair_sums_lanes<L>(C, i, gt & (L - 1), G.n, p, v, pos, vel, cs, nl, nn);
+    }
     if (L > 1 && (gt & (L - 1)) != 0) return;
     if (sums) {  // reverse mode keeps the sums for the pullback of this step
         sums[i] = make_float4(S.ax, S.ay, S.az, 0.0f);
@@ -605,7 +638,7 @@ __global__ __launch_bounds__(256) void voxel_force_kernel(
             if (t0 + u >= cnt || jj[u] == i) continue;
             const float4 q = qq[u], vj = vv[u];
             const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
-            const float r = sqrtf(dx * dx + dy * dy + dz * dz);
+            const float r = sqrtf(norm2(dx, dy, dz));
             const float hr = C.h - r;
             // voxel_kernels.py:162-168: (p_i/rho_i^2 + p_j/rho_j^2) * grad W
             const float cp = (fi + q.w * vj.w * vj.w) * C.grad_c * hr * hr * (1.0f / r);
@@ -792,6 +825,23 @@ constexpr int kDiagBlocks = 512;
 // particle does (1.36 against 1.92 ms per step).
 constexpr int64_t kFarParticles = int64_t(1) << 20;
 
+// Lanes that share a particle in the density and force passes of a plain context with one lane
+// per particle, summing in its order: one lane leaves the card idle on few particles.  us per
+// launch, density / force, with one lane, 8 and 16 (h for about 30 neighbours in the box, 105
+// in the reference's run):
+//     4,096 particles   44 / 12      14 /  9      12 /  7
+//    16,384             42 / 11      17 /  9      17 /  9
+//    20,000 reference  114 / 142     32 / 25      25 / 21
+//    40,000 reference  196 / 249     86 / 93      61 / 95
+//    32,768             39 / 11      18 / 10      24 / 12
+//    65,536             41 / 11      30 / 14      30 / 17
+//    98,304             49 / 14      40 / 17      39 / 22
+//   131,072             45 / 16      56 / 22      78 / 30
+int ordered_lanes(const sph_ctx* c) {
+    if (c->lanes != 1 || !c->inst.empty() || c->sc.formulation != SPH_FORM_NAIVE) return 1;
+    return c->n <= 24576 ? 16 : c->n <= 98304 ? 8 : 1;
+}
+
 hipError_t launch_fill_u32(uint32_t* p, uint32_t v, int64_t n, hipStream_t s) {
     if (n > 0) fill_u32_kernel<<<blocks_for(n, 256), 256, 0, s>>>(p, v, n);
     return hipGetLastError();
@@ -829,11 +879,11 @@ hipError_t launch_rekey(sph_ctx* c, hipStream_t s) {
     return hipGetLastError();
 }
 
-template <int L, bool FAR = false>
+template <int L, bool FAR = false, bool ORDERED = false>
 void launch_density_lanes(sph_ctx* c, hipStream_t s) {
     const int bs = c->density_block;
     const Buffers& b = c->b;
-    naive_density_kernel<L, FAR><<<blocks_for(c->n * L, bs), bs, 0, s>>>(c->sc, b.posA, b.velA, b.cs, b.rhoA, b.nl, b.nn);
+    naive_density_kernel<L, FAR, ORDERED><<<blocks_for(c->n * L, bs), bs, 0, s>>>(c->sc, b.posA, b.velA, b.cs, b.rhoA, b.nl, b.nn);
 }
 
 hipError_t launch_density(sph_ctx* c, hipStream_t s) {
@@ -859,17 +909,22 @@ hipError_t launch_density(sph_ctx* c, hipStream_t s) {
         case 32: launch_density_lanes<32>(c, s); break;
         case 64: launch_density_lanes<64>(c, s); break;
         default:
-            if (c->n > kFarParticles) launch_density_lanes<1, true>(c, s);
-            else launch_density_lanes<1>(c, s);
+            switch (ordered_lanes(c)) {
+                case 16: launch_density_lanes<16, false, true>(c, s); break;
+                case 8: launch_density_lanes<8, false, true>(c, s); break;
+                default:
+                    if (c->n > kFarParticles) launch_density_lanes<1, true>(c, s);
+                    else launch_density_lanes<1>(c, s);
+            }
             break;
     }
     return hipGetLastError();
 }
 
-template <int MODE, int L, bool COUNT = false>
+template <int MODE, int L, bool COUNT = false, bool ORDERED = false>
 void launch_force_lanes(sph_ctx* c, hipStream_t s, float4* dP, float4* dV, float4* dF) {
     const int bs = c->force_block;
-    naive_force_kernel<MODE, L, COUNT><<<blocks_for(c->n * L, bs), bs, 0, s>>>(
+    naive_force_kernel<MODE, L, COUNT, ORDERED><<<blocks_for(c->n * L, bs), bs, 0, s>>>(
         c->sc, c->b.posA, c->b.velA, c->b.pidA, c->b.rhoA, c->b.cs, c->b.nl, c->b.nn, c->b.posB, c->b.velB,
         c->b.pidB, c->b.keyI, c->b.valI, c->b.rng, c->b.pipe, dP, dV, dF, c->b.flags, c->b.sums,
         COUNT ? c->b.cell_cnt : nullptr, COUNT ? c->b.keyS[0] : nullptr,
@@ -903,7 +958,13 @@ void launch_force_mode(sph_ctx* c, hipStream_t s, bool count) {
             case 16: launch_force_lanes<MODE, 16, true>(c, s, dP, dV, dF); break;
             case 32: launch_force_lanes<MODE, 32, true>(c, s, dP, dV, dF); break;
             case 64: launch_force_lanes<MODE, 64, true>(c, s, dP, dV, dF); break;
-            default: launch_force_lanes<MODE, 1, true>(c, s, dP, dV, dF); break;
+            default:
+                switch (ordered_lanes(c)) {
+                    case 16: launch_force_lanes<MODE, 16, true, true>(c, s, dP, dV, dF); break;
+                    case 8: launch_force_lanes<MODE, 8, true, true>(c, s, dP, dV, dF); break;
+                    default: launch_force_lanes<MODE, 1, true>(c, s, dP, dV, dF);
+                }
+                break;
         }
         return;
     }
@@ -914,7 +975,13 @@ void launch_force_mode(sph_ctx* c, hipStream_t s, bool count) {
         case 16: launch_force_lanes<MODE, 16>(c, s, dP, dV, dF); break;
         case 32: launch_force_lanes<MODE, 32>(c, s, dP, dV, dF); break;
         case 64: launch_force_lanes<MODE, 64>(c, s, dP, dV, dF); break;
-        default: launch_force_lanes<MODE, 1>(c, s, dP, dV, dF); break;
+        default:
+            switch (ordered_lanes(c)) {
+                case 16: launch_force_lanes<MODE, 16, false, true>(c, s, dP, dV, dF); break;
+                case 8: launch_force_lanes<MODE, 8, false, true>(c, s, dP, dV, dF); break;
+                default: launch_force_lanes<MODE, 1>(c, s, dP, dV, dF);
+            }
+            break;
     }
 }
 
@@ -922,7 +989,7 @@ bool count_in_force(const sph_ctx* c) {
     return c->cell_sort && c->inst.empty() && c->sc.formulation == SPH_FORM_NAIVE && cell_sort_global(c);
 }
 
-bool tile_sums_in_force(const sph_ctx* c) { return count_in_force(c) && c->lanes == 1; }
+bool tile_sums_in_force(const sph_ctx* c) { return count_in_force(c) && c->lanes == 1 && ordered_lanes(c) == 1; }
 
 hipError_t launch_force(sph_ctx* c, hipStream_t s, bool count) {
     if (c->n == 0) return hipGetLastError();

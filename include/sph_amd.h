@@ -224,7 +224,9 @@ int sph_set_launch(sph_ctx* ctx, int32_t density_block, int32_t force_block);
 /* Lanes of a wavefront that share one particle in the NAIVE density and force passes
  * (1, 2, 4, 8, 16, 32 or 64; default 1), for the autotuner: small or dense problems (few particles,
  * many neighbours each) get that many times the parallelism.  The neighbour lists are the
- * same for every value; sums are added in a different order (FP32 rounding only).  The
+ * same for every value; sums are added in a different order (FP32 rounding only).  With 1, a
+ * plain context of few particles still shares each among several lanes, which add its sums in
+ * one lane's order, to the same bits.  The
  * reference launches one thread per particle (thread_layout.py:27-33).  On a batched
  * context every instance gets `lanes`. */
 int sph_set_lanes(sph_ctx* ctx, int32_t lanes);
