@@ -454,6 +454,99 @@ int read_nonfinite(sph_ctx* c, hipStream_t s, int64_t* count) {
     return SPH_OK;
 }
 
+// The copies of sph_advance_host between the caller's arrays and the device staging, whose
+// image is kStagingHead bytes (the non-finite count in the first word), then pos, vel and
+// rho.  They go through the caller's page-locked memory: in one piece where it holds the
+// image, else in pieces through its two halves by turns, so that a piece is copied on the host
+// while the next one crosses the bus.
+constexpr size_t kStagingHead = 256;
+
+struct HostCopy {
+    char* pin = nullptr;
+    size_t half = 0, n = 0;
+    bool whole = false;
+    hipStream_t s = nullptr;
+    hipEvent_t ev[2] = {nullptr, nullptr};
+    bool used[2] = {false, false};
+
+    ~HostCopy() {
+        for (auto e : ev)
+            if (e) (void)hipEventDestroy(e);
+    }
+    int open(void* pinned, size_t bytes, size_t count, hipStream_t stream) {
+        pin = (char*)pinned;
+        n = count;
+        s = stream;
+        whole = kStagingHead + 56 * n <= bytes;
+        half = (bytes / 2) & ~(size_t)255;
+        int rc = SPH_OK;
+        for (int k = 0; k < 2 && !whole && rc == SPH_OK; ++k)
+            rc = hip_check(hipEventCreateWithFlags(&ev[k], hipEventDisableTiming), "create event");
+        return rc;
+    }
+    // bytes [o, o + len) of the image from (OUT: to) the caller's arrays
+    template <bool OUT, typename T>
+    void move(char* piece, size_t o, size_t len, T* const (&arrays)[3]) const {
+        const size_t begin[4] = {kStagingHead, kStagingHead + 24 * n, kStagingHead + 48 * n, kStagingHead + 56 * n};
+        for (int a = 0; a < 3; ++a) {
+            const size_t lo = std::max(o, begin[a]), hi = std::min(o + len, begin[a + 1]);
+            if (lo >= hi || !arrays[a]) continue;
+            char* const mine = (char*)arrays[a] + (lo - begin[a]);
+            if (OUT) memcpy(mine, piece + (lo - o), hi - lo);
+            else memcpy(piece + (lo - o), mine, hi - lo);
+        }
+    }
+    int to_device(char* dev, const double* pos, const double* vel) {
+        const double* const in[3] = {pos, vel, nullptr};
+        const size_t end = kStagingHead + 48 * n, step = whole ? end : half;
+        int rc;
+        for (size_t o = kStagingHead, k = 0; o < end; o += step, ++k) {
+            const size_t len = std::min(step, end - o);
+            char* const piece = pin + (whole ? o : (k & 1) * half);
+            if (used[k & 1] && (rc = hip_check(hipEventSynchronize(ev[k & 1]), "wait for a piece"))) return rc;
+            move<false>(piece, o, len, in);
+            if ((rc = hip_check(hipMemcpyAsync(dev + o, piece, len, hipMemcpyHostToDevice, s), "copy state in"))) return rc;
+            if (!whole) {
+                if ((rc = hip_check(hipEventRecord(ev[k & 1], s), "record event"))) return rc;
+                used[k & 1] = true;
+            }
+        }
+        return SPH_OK;
+    }
+    // waits for the stream; check: fails if the image's count is not zero
+    int to_host(const char* dev, double* pos, double* vel, double* rho, bool check) {
+        double* const out[3] = {pos, vel, rho};
+        const size_t end = kStagingHead + 56 * n, step = whole ? end : half;
+        const size_t pieces = (end + step - 1) / step;
+        uint32_t found = 0;
+        int rc = SPH_OK;
+        for (size_t k = 0; k < pieces + (whole ? 0 : 1) && rc == SPH_OK; ++k) {
+            if (k < pieces) {
+                const size_t o = k * step, len = std::min(step, end - o);
+                rc = hip_check(hipMemcpyAsync(pin + (whole ? 0 : (k & 1) * half), dev + o, len, hipMemcpyDeviceToHost, s),
+                               "copy state out");
+                if (rc == SPH_OK && !whole) rc = hip_check(hipEventRecord(ev[k & 1], s), "record event");
+            }
+            if (rc != SPH_OK || (!whole && k == 0)) continue;
+            const size_t p = whole ? k : k - 1, o = p * step, len = std::min(step, end - o);
+            rc = whole ? hip_check(hipStreamSynchronize(s), "wait for the state")
+                       : hip_check(hipEventSynchronize(ev[p & 1]), "wait for a piece");
+            if (rc != SPH_OK) break;
+            char* const piece = pin + (whole ? 0 : (p & 1) * half);
+            if (p == 0 && check && n > 0) memcpy(&found, piece, sizeof(found));
+            if (found == 0) move<true>(piece, o, len, out);
+        }
+        if (rc != SPH_OK) {
+            (void)hipStreamSynchronize(s);  // nothing may still write to the caller's memory
+            return rc;
+        }
+        if (found != 0)
+            return fail(SPH_E_NONFINITE, "%u particle positions were NaN or infinite when hashed (since the last check)",
+                        found);
+        return SPH_OK;
+    }
+};
+
 void assign_buffers(sph_ctx* c, void* dev);
 
 int ready(const sph_ctx* c, bool need_state) {
@@ -734,6 +827,44 @@ int sph_download_state_f32(sph_ctx* c, float* x, float* y, float* z, float* vx, 
     int rc = ready(c, true);
     if (rc) return rc;
     return hip_check(sph::launch_download_f32(c, x, y, z, vx, vy, vz, rho, (hipStream_t)stream), "download");
+}
+
+size_t sph_host_staging_bytes(const sph_ctx* c) { return c ? kStagingHead + 56 * (size_t)(c->n > 0 ? c->n : 1) : 0; }
+
+int sph_advance_host(sph_ctx* c, int32_t nsteps, const double* pos, const double* vel, double* pos_out,
+                     double* vel_out, double* rho_out, void* dev_staging, size_t dev_bytes, void* pinned,
+                     size_t pinned_bytes, void* stream) {
+    int rc = ready(c, !pos && !vel);
+    if (rc) return rc;
+    if ((pos == nullptr) != (vel == nullptr)) return fail(SPH_E_INVALID, "one of pos and vel is null");
+    if (c->n > 0 && (!pos_out || !vel_out || !rho_out)) return fail(SPH_E_INVALID, "null output");
+    if (nsteps < 0) return fail(SPH_E_INVALID, "nsteps < 0");
+    if (!dev_staging || dev_bytes < sph_host_staging_bytes(c) || ((uintptr_t)dev_staging & 255u))
+        return fail(SPH_E_INVALID, "staging of %zu bytes, %zu needed (256-byte aligned)", dev_bytes, sph_host_staging_bytes(c));
+    if (!pinned || pinned_bytes < 4096 || ((uintptr_t)pinned & 255u))
+        return fail(SPH_E_INVALID, "pinned memory of %zu bytes, 4096 needed (256-byte aligned)", pinned_bytes);
+    if (!pos && c->last_stage != 0 && c->last_stage != SPH_STAGE_FORCE)
+        return fail(SPH_E_STATE, "a staged step is in progress (run it to SPH_STAGE_FORCE first)");
+    hipStream_t s = (hipStream_t)stream;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if ((rc = hip_check(hipStreamIsCapturing(s, &st), "capture status"))) return rc;
+    if (st != hipStreamCaptureStatusNone) return fail(SPH_E_STATE, "sph_advance_host waits for its copies: not under capture");
+    const size_t n = (size_t)c->n;
+    char* const dev = (char*)dev_staging;
+    double* const dpos = (double*)(dev + kStagingHead);
+    double* const dvel = dpos + 3 * n;
+    HostCopy copy;
+    if ((rc = copy.open(pinned, pinned_bytes, n, s))) return rc;
+    if (pos) {
+        if ((rc = copy.to_device(dev, pos, vel))) return rc;
+        if ((rc = sph_upload_state(c, dpos, dvel, stream))) return rc;
+    }
+    if ((rc = run_steps(c, s, nsteps))) return rc;
+    const bool check = c->check_finite && nsteps > 0;
+    if ((rc = hip_check(sph::launch_download_f64(c, dpos, dvel, dvel + 3 * n, nullptr, s, check ? (uint32_t*)dev : nullptr),
+                        "download")))
+        return rc;
+    return copy.to_host(dev, pos_out, vel_out, rho_out, check);
 }
 
 int64_t sph_buffer_elems(const sph_ctx* c, int32_t which) {

@@ -248,7 +248,9 @@ hipError_t launch_density(sph_ctx* c, hipStream_t s);
 // count: also rank the new keys into cell_cnt / keyS[0] (count_in_force) and add them to the
 // tile sums in cell_part array part_phase (tile_sums_in_force), for the next sort
 hipError_t launch_force(sph_ctx* c, hipStream_t s, bool count = false);
-hipError_t launch_download_f64(sph_ctx* c, double* pos, double* vel, double* rho, double* force, hipStream_t s);
+// found: if given (device), receives the count of non-finite positions, which is cleared
+hipError_t launch_download_f64(sph_ctx* c, double* pos, double* vel, double* rho, double* force, hipStream_t s,
+                               uint32_t* found = nullptr);
 hipError_t launch_download_f32(sph_ctx* c, float* x, float* y, float* z, float* vx, float* vy, float* vz,
                                float* rho, hipStream_t s);
 hipError_t launch_read_buffer(sph_ctx* c, int which, void* out, hipStream_t s);

@@ -659,15 +659,21 @@ __global__ __launch_bounds__(256) void voxel_force_kernel(
 }
 
 // ---------------------------------------------------------------------------------------
-// Boundary output: scatter from cell order back to particle order.
+// Boundary output: scatter from cell order back to particle order.  found: if given, takes the
+// count of non-finite positions, which is cleared.
 // ---------------------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void download_f64_kernel(int n, const float4* __restrict__ posB,
                                                             const float4* __restrict__ velB,
                                                             const uint32_t* __restrict__ pidB,
                                                             const float4* __restrict__ dbgF, double* __restrict__ pos,
                                                             double* __restrict__ vel, double* __restrict__ rho,
-                                                            double* __restrict__ force) {
+                                                            double* __restrict__ force, uint32_t* __restrict__ flags,
+                                                            uint32_t* __restrict__ found) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == 0 && found) {
+        *found = flags[kFlagNonFinite];
+        flags[kFlagNonFinite] = 0u;
+    }
     if (i >= n) return;
     const float4 p = posB[i], v = velB[i];
     const int64_t id = pidB[i];
@@ -999,10 +1005,11 @@ hipError_t launch_force(sph_ctx* c, hipStream_t s, bool count) {
     return hipGetLastError();
 }
 
-hipError_t launch_download_f64(sph_ctx* c, double* pos, double* vel, double* rho, double* force, hipStream_t s) {
+hipError_t launch_download_f64(sph_ctx* c, double* pos, double* vel, double* rho, double* force, hipStream_t s,
+                               uint32_t* found) {
     if (c->n > 0)
         download_f64_kernel<<<blocks_for(c->n, 256), 256, 0, s>>>((int)c->n, c->b.posB, c->b.velB, c->b.pidB,
-                                                                    c->b.dbgF, pos, vel, rho, force);
+                                                                    c->b.dbgF, pos, vel, rho, force, c->b.flags, found);
     return hipGetLastError();
 }
 

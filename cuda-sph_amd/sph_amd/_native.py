@@ -64,7 +64,12 @@ EXPORTED = [
     "sph_create_batch", "sph_batch_info", "sph_set_constants", "sph_set_lanes", "sph_adjoint_seed", "sph_adjoint_step",
     "sph_adjoint_read", "sph_set_batch_lanes", "sph_adjoint_snapshot_bytes", "sph_adjoint_save", "sph_step_save", "sph_adjoint_step_from",
     "sph_check_finite", "sph_noalloc_scratch_bytes", "sph_step_noalloc", "sph_step_timed", "sph_set_slabs",
+    "sph_host_staging_bytes", "sph_advance_host",
 ]
+
+# Page-locked memory a context's advance_host keeps at most; a larger state goes through it in
+# pieces.
+PINNED_BYTES = 16 << 20
 
 _lib = None
 
@@ -90,6 +95,8 @@ def load_library() -> ctypes.CDLL:
         "sph_upload_state_f32": ([vp] + [vp] * 6 + [vp], i32),
         "sph_step": ([vp, i32, vp], i32),
         "sph_step_timed": ([vp, i32, POINTER(ctypes.c_double), vp], i32),
+        "sph_host_staging_bytes": ([vp], c_size_t),
+        "sph_advance_host": ([vp, i32, vp, vp, vp, vp, vp, vp, c_size_t, vp, c_size_t, vp], i32),
         "sph_download_state": ([vp, vp, vp, vp, vp, vp], i32),
         "sph_download_state_f32": ([vp] + [vp] * 7 + [vp], i32),
         "sph_run_stage": ([vp, i32, vp], i32),
@@ -185,6 +192,7 @@ class NativeContext:
         self._ws = torch.empty(nbytes + 256, dtype=torch.uint8, device=self.device)
         off = (-self._ws.data_ptr()) % 256
         self.workspace_bytes = nbytes
+        self._staging = None  # device and page-locked memory of advance_host
         with torch.cuda.device(self.device):
             check(self.lib.sph_bind_workspace(h, c_void_p(self._ws.data_ptr() + off), nbytes, _stream(self.device)),
                   "sph_bind_workspace")
@@ -219,6 +227,28 @@ class NativeContext:
     def step(self, nsteps: int = 1):
         self.generation += 1
         check(self.lib.sph_step(self.handle, int(nsteps), _stream(self.device)), "sph_step")
+
+    def advance_host(self, state, nsteps: int):
+        """nsteps steps from a host state (pos, vel: contiguous float64 (N, 3) arrays; None: the
+        resident state) to a host state: new float64 arrays pos (N, 3), vel (N, 3), rho (N,).
+        Waits for the stream and raises like step() on a context that checks its state."""
+        if self._staging is None:
+            nbytes = int(self.lib.sph_host_staging_bytes(self.handle))
+            dev = torch.empty(nbytes + 256, dtype=torch.uint8, device=self.device)
+            size = min((nbytes + 255) // 256 * 256, PINNED_BYTES)
+            pin = torch.empty(max(size, 4096) + 256, dtype=torch.uint8, pin_memory=True)
+            self._staging = (dev, dev.data_ptr() + (-dev.data_ptr()) % 256, nbytes,
+                             pin, pin.data_ptr() + (-pin.data_ptr()) % 256, max(size, 4096))
+        _, dptr, dbytes, _, pptr, pbytes = self._staging
+        n = self.n
+        out = np.empty((n, 3)), np.empty((n, 3)), np.empty(n)
+        pos, vel = (None, None) if state is None else (state[0].ctypes.data, state[1].ctypes.data)
+        self.generation += 1
+        with torch.cuda.device(self.device):
+            check(self.lib.sph_advance_host(self.handle, int(nsteps), pos, vel, out[0].ctypes.data, out[1].ctypes.data,
+                                            out[2].ctypes.data, dptr, dbytes, pptr, pbytes, _stream(self.device)),
+                  "sph_advance_host")
+        return out
 
     def step_timed(self, nsteps: int) -> dict:
         """step(nsteps) with HIP events between the stages (waits for them): mean ms per step

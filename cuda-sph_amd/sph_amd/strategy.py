@@ -90,18 +90,18 @@ class SPHStrategy:
 
     # -- reference entry point -----------------------------------------------------------
     def compute_next_state(self, old_state: SimulationState) -> SimulationState:
-        self.old_state = old_state
-        self._initialize_computation()
-        self.ctx.step(1)
-        self._finalize_computation()
-        return self.new_state
+        return self.advance(old_state, 1)
 
     def advance(self, state: SimulationState, nsteps: int) -> SimulationState:
         """nsteps steps with one upload and one download."""
         self.old_state = state
-        self._initialize_computation()
-        self.ctx.step(int(nsteps))
-        self._finalize_computation()
+        if self.keep_terms:
+            self._initialize_computation()
+            self.ctx.step(int(nsteps))
+            self._finalize_computation()
+        else:
+            # copies, steps and the finite check in one call, through page-locked memory
+            self._returned(self.ctx.advance_host(self._new_arrays(), int(nsteps)))
         return self.new_state
 
     def capture(self, nsteps: int) -> torch.cuda.CUDAGraph:
@@ -119,28 +119,37 @@ class SPHStrategy:
         return g
 
     # -- stages --------------------------------------------------------------------------
+    def _new_arrays(self):
+        """Position and velocity arrays of the state to step from, or None when the device holds
+        that state already: it is the one this strategy returned last."""
+        st = self.old_state
+        if st is not None and st is self.new_state and self.ctx.generation == self._returned_generation:
+            return None
+        pos = np.ascontiguousarray(st.position, dtype=np.float64)
+        vel = np.ascontiguousarray(st.velocity, dtype=np.float64)
+        if pos.shape != (self.ctx.n, 3) or vel.shape != (self.ctx.n, 3):
+            raise ValueError(f"state arrays must be ({self.ctx.n}, 3), got {pos.shape} / {vel.shape}")
+        return pos, vel
+
     def _initialize_computation(self):
         """Host-to-device copy of the state (abstract_sph_strategy.py:64-74), skipped when the
         state is the one this strategy returned last."""
-        st = self.old_state
-        if st is not None and st is self.new_state and self.ctx.generation == self._returned_generation:
-            return
-        pos = torch.from_numpy(np.ascontiguousarray(st.position, dtype=np.float64)).to(self.device)
-        vel = torch.from_numpy(np.ascontiguousarray(st.velocity, dtype=np.float64)).to(self.device)
-        if pos.shape != (self.ctx.n, 3) or vel.shape != (self.ctx.n, 3):
-            raise ValueError(f"state arrays must be ({self.ctx.n}, 3), got {tuple(pos.shape)} / {tuple(vel.shape)}")
-        self.ctx.upload(pos, vel)
+        arrays = self._new_arrays()
+        if arrays is not None:
+            self.ctx.upload(*[torch.from_numpy(a).to(self.device) for a in arrays])
+
+    def _returned(self, host) -> None:
+        for a in host:
+            a.setflags(write=False)
+        self.new_state = SimulationState(*host)
+        self._returned_generation = self.ctx.generation
 
     def _finalize_computation(self):
         """Device-to-host copy into a new SimulationState (abstract_sph_strategy.py:76-84)."""
         out = self.ctx.download(force=self.keep_terms)
-        host = [t.cpu().numpy() for t in out[:3]]
-        for a in host:
-            a.setflags(write=False)
         if self.keep_terms:
             self.result_force = out[3].cpu().numpy()
-        self.new_state = SimulationState(host[0], host[1], host[2])
-        self._returned_generation = self.ctx.generation
+        self._returned([t.cpu().numpy() for t in out[:3]])
 
     def diagnostics(self) -> dict:
         """FP64 totals of the resident state."""

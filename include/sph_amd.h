@@ -16,8 +16,8 @@
  *     Pointers without the prefix are host pointers.
  *   - stream is a hipStream_t passed as void*; NULL means the default stream.  All work
  *     is enqueued on that stream; the calls that wait for it are sph_bind_workspace,
- *     sph_set_batch_lanes, sph_check_finite, sph_step_timed and sph_step on a context
- *     created with SPH_FLAG_CHECK_FINITE.
+ *     sph_set_batch_lanes, sph_check_finite, sph_step_timed, sph_advance_host and sph_step on
+ *     a context created with SPH_FLAG_CHECK_FINITE.
  *   - The library never allocates device memory: the caller allocates the workspace
  *     (sph_workspace_bytes) and keeps it alive while the context is used.
  *   - A context is not re-entrant: calls on one context must not overlap.
@@ -161,6 +161,20 @@ int sph_download_state(sph_ctx* ctx, double* dev_pos, double* dev_vel, double* d
 /* Same as sph_download_state into float32 structure-of-arrays outputs (any may be NULL). */
 int sph_download_state_f32(sph_ctx* ctx, float* dev_x, float* dev_y, float* dev_z, float* dev_vx, float* dev_vy,
                            float* dev_vz, float* dev_rho, void* stream);
+
+/* sph_upload_state, sph_step and sph_download_state for a caller whose state is in host
+ * memory: the whole of compute_next_state (abstract_sph_strategy.py:31-46) in one call, with
+ * one host-to-device and one device-to-host copy.  pos, vel: host float64 (N, 3), or both
+ * NULL to go on from the resident state.  pos_out, vel_out (N, 3) and rho_out (N): host
+ * float64, written when the call succeeds (also not when it returns SPH_E_NONFINITE; the
+ * check is sph_step's).  dev_staging: device memory of at least sph_host_staging_bytes
+ * bytes (256-byte aligned); pinned: page-locked host memory of pinned_bytes bytes, at least
+ * 4,096 (256-byte aligned), through which the copies go, in two halves by turns where it is smaller than
+ * the state.  Waits for the stream; not under graph capture. */
+size_t sph_host_staging_bytes(const sph_ctx* ctx);
+int sph_advance_host(sph_ctx* ctx, int32_t nsteps, const double* pos, const double* vel, double* pos_out,
+                     double* vel_out, double* rho_out, void* dev_staging, size_t dev_bytes, void* pinned,
+                     size_t pinned_bytes, void* stream);
 
 /* Stage-by-stage execution of one step, for parity tests and profiling.  The stages in
  * order; sph_step(ctx, 1) runs exactly this sequence.
