@@ -34,6 +34,8 @@
 // The per-slot passes (count, scatter, order) map workgroups to slot ranges XCD by XCD as
 // the density and force passes do (xcd_tile), so each XCD reads back from its own L2 the keys
 // and state its force pass wrote (step 0.2245 -> 0.2226 ms on the 1M dam break).
+#include <algorithm>
+
 #include "sph_device.h"
 
 namespace sph {
@@ -63,6 +65,24 @@ struct SlabTable {
         return f;
     }
 };
+
+// The fields of an occupied cell of count particles, b_j of them in slabs below j: the offsets of
+// slabs 1 .. S - 1, each stored + 1, none if the largest does not fit; the count + 1 where it
+// fits.
+__device__ __forceinline__ uint32_t slab_fields(const SlabTable& T, uint32_t b1, uint32_t b2, uint32_t b3,
+                                                uint32_t count) {
+    const bool four = T.shift == 2;
+    const uint32_t top = four ? b3 : b1;
+    uint32_t fields = 0u;
+    if (top + 1u <= (1u << T.bits) - 1u) {
+        fields = (b1 + 1u) << T.start_bits;
+        if (four) fields |= ((b2 + 1u) << (T.start_bits + T.bits)) | ((b3 + 1u) << (T.start_bits + 2 * T.bits));
+    }
+    if (T.count_bits > 0 && count + 1u <= (1u << T.count_bits) - 1u) fields |= (count + 1u) << T.count_pos;
+    return fields;
+}
+
+constexpr uint32_t kIdMask = kCellKeyMask;  // particle ids are below 2^27
 
 SlabTable slab_table(const StepConsts& S) {
     return SlabTable{S.slab_shift, S.start_bits, S.slab_bits, S.count_pos, S.count_bits, S.start_mask};
@@ -286,16 +306,7 @@ __global__ __launch_bounds__(CT) void cell_order_kernel(int n, SlabTable T, cons
     }
     const uint32_t f = a + r;
     if (slabs && r == 0u) {
-        // offsets of slabs 1 .. S - 1, each stored + 1, none if the largest does not fit; the
-        // count + 1 where it fits
-        const bool four = T.shift == 2;
-        const uint32_t top = four ? b3 : b1;
-        uint32_t fields = 0u;
-        if (top + 1u <= (1u << T.bits) - 1u) {
-            fields = (b1 + 1u) << T.start_bits;
-            if (four) fields |= ((b2 + 1u) << (T.start_bits + T.bits)) | ((b3 + 1u) << (T.start_bits + 2 * T.bits));
-        }
-        if (T.count_bits > 0 && (b - a) + 1u <= (1u << T.count_bits) - 1u) fields |= ((b - a) + 1u) << T.count_pos;
+        const uint32_t fields = slab_fields(T, b1, b2, b3, b - a);
         if (fields) cs[k] = a | fields;
     }
     skey[f] = k;
@@ -307,56 +318,217 @@ __global__ __launch_bounds__(CT) void cell_order_kernel(int n, SlabTable T, cons
     }
 }
 
-// Small problems (at most kLdsSortCells cells and kLdsSortMax particles): count, scan and
-// scatter in one workgroup with the counts in LDS, in place of the four kernels above, whose
-// launches dominate at these sizes.  The LDS atomics rank the particles of a cell in an
-// arbitrary order, as the global ones do; cell_order_kernel makes the order.  The global
-// per-cell counts are not used (they stay zero).  Measured on 4,096 particles: 20.2 against
-// 23.1 us per step with 4,096 cells; with 32,768 cells (or 16,384 particles) the one
-// workgroup's sweep costs more than the launches it saves.
-constexpr int LT = 1024;                // threads of the one workgroup
-constexpr int kLdsSortCells = 8192;
-constexpr int kLdsSortMax = 8192;
-constexpr int LWAVES = LT / 64;
+// Few particles: the whole sort in one launch.  Every workgroup owns a contiguous range of cells:
+// it reads all keys, counts those below its range (where its part of the order begins) and
+// collects those in it, scans its cells' counts, places its particles cell by cell in LDS,
+// orders each cell there and gathers its part of the state, and writes its part of the table.
+// The passes above take five launches of about 4.4 us each at these sizes, whatever their work,
+// and atomics in the force pass; this one takes 6 us with 4,096 particles (two launches before,
+// 12.4), 8 with 16,384 (23), 12 with 65,537 (18).  What bounds it is one latency after another
+// (keys, ids, state), and for many particles the keys' 4 n bytes in each of 256 workgroups.
+// A range with more than kOneList particles is collected in global memory (tmpE, tmpK) instead,
+// by a second walk over the keys.  A cell of more than kHeavyCell particles is ordered through a
+// bitmap of its (slab, id) in place of comparing each with each, which one workgroup alone
+// would take long for (70,000 particles in one cell: 5e9 comparisons).
+constexpr int OT = 1024;
+constexpr int OWAVES = OT / 64;
+constexpr int kOneGroups = 256;  // one per CU
+constexpr int kOneList = 2048;   // particles of a workgroup's range kept in LDS
+constexpr int kOneCells = 4096;  // cells of a range, at most
+constexpr int kOneLoads = 4;     // 16-byte key loads in flight per lane
+constexpr int kHeavyCell = 512;
+// step with the passes above against this one (30 neighbours, 4 lanes): 30.6 against 25.4 us with
+// 16,384 particles, 40.6 / 38.6 with 49,152, 45.3 / 44.6 with 65,537, 51.3 / 51.9 with 81,920
+constexpr int64_t kOneSort = 73728;
+constexpr int kHeavyMost = (int)(kOneSort / (kHeavyCell + 1)) + 1;  // heavy cells of a range, at most
+inline __host__ __device__ int heavy_words(int n, bool slabs) { return ((slabs ? 4 : 1) * n + 31) / 32; }
 
-__global__ __launch_bounds__(LT) void cell_sort_lds_kernel(int n, int m, const uint32_t* __restrict__ keyI,
-                                                           uint32_t* __restrict__ rank, uint32_t* __restrict__ cs,
-                                                           uint32_t* __restrict__ tmp, SlabTable T) {
-    __shared__ uint32_t cnt[kLdsSortCells + kLdsSortCells / 32];  // index c at cpad(c)
-    __shared__ uint32_t lw[LWAVES];
-    for (int c = threadIdx.x; c < m; c += LT) cnt[cpad(c)] = 0u;
+template <bool GATHER>
+__global__ __launch_bounds__(OT) void cell_sort_one_kernel(
+    int n, int m, int per, SlabTable T, const uint32_t* __restrict__ keyI, const uint32_t* __restrict__ pidB,
+    uint32_t* __restrict__ cs, uint32_t* __restrict__ skey, uint32_t* __restrict__ sval,
+    const float4* __restrict__ posB, const float4* __restrict__ velB, float4* __restrict__ posA,
+    float4* __restrict__ velA, uint32_t* __restrict__ pidA, uint32_t* tmpE, uint32_t* tmpK) {
+    extern __shared__ uint32_t s_one[];
+    uint32_t* const start = s_one;             // per + 1: a cell's first place in the range
+    uint32_t* const cur = start + per + 1;     // per: its count, then its next free place
+    uint32_t* const table = cur + per;         // per: its table entry
+    uint32_t* const listE = table + per;       // kOneList: the range's particles (slots) as found ...
+    uint32_t* const listK = listE + kOneList;  // ... their keys
+    uint32_t* const ordE = listK + kOneList;   // ... cell by cell
+    uint32_t* const ordK = ordE + kOneList;    // ... (slab, id) there
+    uint32_t* const bits = ordK + kOneList;    // heavy_words: a heavy cell's (slab, id)
+    __shared__ uint32_t s_wave[OWAVES], s_count, s_below, s_heavy, s_cell[kHeavyMost], s_ones[OT];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int lo = xcd_tile(blockIdx.x, gridDim.x) * per, hi = min(lo + per, m);  // this range of cells
+    if (lo >= hi) return;
+    const int own = hi - lo;
+    for (int c = tid; c < own; c += OT) cur[c] = 0u;
+    if (tid == 0) s_count = s_below = s_heavy = 0u;
     __syncthreads();
-    for (int i = threadIdx.x; i < n; i += LT) rank[i] = atomicAdd(&cnt[cpad((int)(keyI[i] & kCellKeyMask))], 1u);
+    uint32_t below = 0u;
+    auto cell_of = [&](uint32_t key) { return (int)(key & kCellKeyMask); };
+    auto mine = [&](int c) { return c >= lo && c < hi; };
+    auto take = [&](uint32_t key, int c, int e) {
+        atomicAdd(&cur[c - lo], 1u);
+        const uint32_t at = atomicAdd(&s_count, 1u);
+        if (at < (uint32_t)kOneList) {
+            listE[at] = (uint32_t)e;
+            listK[at] = key;
+        }
+    };
+    // most quads hold no key of the range
+    const uint4* const key4 = reinterpret_cast<const uint4*>(keyI);
+    const int quads = n / 4;
+    for (int v0 = tid; v0 < quads; v0 += kOneLoads * OT) {
+        uint4 k[kOneLoads];
+#pragma unroll
+        for (int u = 0; u < kOneLoads; ++u) k[u] = key4[min(v0 + u * OT, quads - 1)];
+#pragma unroll
+        for (int u = 0; u < kOneLoads; ++u) {
+            const int v = v0 + u * OT;
+            if (v >= quads) break;
+            const int c[4] = {cell_of(k[u].x), cell_of(k[u].y), cell_of(k[u].z), cell_of(k[u].w)};
+            below += (c[0] < lo ? 1u : 0u) + (c[1] < lo ? 1u : 0u) + (c[2] < lo ? 1u : 0u) + (c[3] < lo ? 1u : 0u);
+            if (mine(c[0]) || mine(c[1]) || mine(c[2]) || mine(c[3])) {
+                if (mine(c[0])) take(k[u].x, c[0], 4 * v);
+                if (mine(c[1])) take(k[u].y, c[1], 4 * v + 1);
+                if (mine(c[2])) take(k[u].z, c[2], 4 * v + 2);
+                if (mine(c[3])) take(k[u].w, c[3], 4 * v + 3);
+            }
+        }
+    }
+    for (int e = 4 * quads + tid; e < n; e += OT) {
+        const uint32_t key = keyI[e];
+        const int c = cell_of(key);
+        below += c < lo ? 1u : 0u;
+        if (mine(c)) take(key, c, e);
+    }
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) below += __shfl_xor(below, o);
+    if (lane == 0 && below) atomicAdd(&s_below, below);
     __syncthreads();
-    // exclusive scan: thread t owns the cells [t per, (t + 1) per)
-    const int per = (m + LT - 1) / LT;
-    const int c0 = min((int)threadIdx.x * per, m), c1 = min(c0 + per, m);
-    uint32_t sum = 0;
-    for (int c = c0; c < c1; ++c) sum += cnt[cpad(c)];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const uint32_t base = s_below, count = s_count;
+    // exclusive scan of the counts, thread t the cells [t each, (t + 1) each)
+    const int each = (own + OT - 1) / OT;
+    const int c0 = min(tid * each, own), c1 = min(c0 + each, own);
+    uint32_t sum = 0u;
+    for (int c = c0; c < c1; ++c) sum += cur[c];
     const uint32_t incl = wave_incl_scan(sum);
-    if (lane == 63) lw[w] = incl;
+    if (lane == 63) s_wave[w] = incl;
     __syncthreads();
     uint32_t run = incl - sum;
-    for (int k = 0; k < w; ++k) run += lw[k];
+    for (int k = 0; k < w; ++k) run += s_wave[k];
     const uint32_t empty = T.empty();
     for (int c = c0; c < c1; ++c) {
-        const uint32_t v = cnt[cpad(c)];
-        cnt[cpad(c)] = run | (v == 0u ? empty : 0u);
+        const uint32_t v = cur[c];
+        start[c] = run;
+        table[c] = (base + run) | (v == 0u ? empty : 0u);
+        cur[c] = run;
         run += v;
+        if (v > (uint32_t)kHeavyCell) s_cell[atomicAdd(&s_heavy, 1u)] = (uint32_t)c;
     }
+    if (tid == 0) start[own] = count;
     __syncthreads();
-    for (int c = threadIdx.x; c < m; c += LT) cs[c] = cnt[cpad(c)];
-    if (threadIdx.x == 0) cs[m] = (uint32_t)n;
-    for (int i = threadIdx.x; i < n; i += LT)
-        tmp[(cnt[cpad((int)(keyI[i] & kCellKeyMask))] & T.start_mask) + rank[i]] = (uint32_t)i;
+    // the range's particles cell by cell in E and K, then each one's place in its cell: the number
+    // of the cell's particles before it
+    const bool slabs = GATHER && T.shift > 0;
+    auto order = [&](uint32_t* E, uint32_t* K, bool listed) {
+        auto place = [&](uint32_t key, uint32_t e) {
+            const uint32_t at = atomicAdd(&cur[cell_of(key) - lo], 1u);
+            E[at] = e;
+            // ids are below 2^27, so the slab bits of a key above the id order both
+            K[at] = (slabs ? key & ~kCellKeyMask : 0u) | pidB[e];
+        };
+        if (listed) {
+            for (uint32_t at = tid; at < count; at += OT) place(listK[at], listE[at]);
+        } else {
+            for (int e = tid; e < n; e += OT) {
+                const uint32_t key = keyI[e];
+                if (mine(cell_of(key))) place(key, (uint32_t)e);
+            }
+            __threadfence_block();
+        }
+        __syncthreads();
+        // particle E[at] of cell c: r of its particles come before it, b_j are in slabs below j
+        auto put = [&](uint32_t at, int c, uint32_t r, uint32_t b1, uint32_t b2, uint32_t b3) {
+            const uint32_t e = E[at], f = base + start[c] + r;
+            if (slabs && r == 0u) table[c] |= slab_fields(T, b1, b2, b3, start[c + 1] - start[c]);
+            skey[f] = (uint32_t)(c + lo);
+            if (!GATHER) sval[f] = e;
+            if (GATHER) {
+                posA[f] = posB[e];
+                velA[f] = velB[e];
+                pidA[f] = K[at] & kIdMask;
+            }
+        };
+        for (uint32_t at = tid; at < count; at += OT) {
+            const uint32_t rank = K[at];
+            const int c = cell_of(keyI[E[at]]) - lo;
+            const uint32_t a = start[c], b = start[c + 1];
+            if (b - a > (uint32_t)kHeavyCell) continue;
+            uint32_t r = 0, b1 = 0, b2 = 0, b3 = 0;
+            for (uint32_t t = a; t < b; ++t) {
+                const uint32_t kt = K[t];
+                r += kt < rank ? 1u : 0u;
+                if (slabs) {
+                    const uint32_t q = kt >> kSlabKeyShift;
+                    b1 += q < 1u ? 1u : 0u;
+                    b2 += q < 2u ? 1u : 0u;
+                    b3 += q < 3u ? 1u : 0u;
+                }
+            }
+            put(at, c, r, b1, b2, b3);
+        }
+        const int words = heavy_words(n, slabs), share = (words + OT - 1) / OT;
+        auto place_of = [&](uint32_t k) { return (slabs ? (k >> kSlabKeyShift) * (uint32_t)n : 0u) + (k & kIdMask); };
+        for (uint32_t h = 0; h < s_heavy; ++h) {
+            const int c = (int)s_cell[h];
+            const uint32_t a = start[c], b = start[c + 1];
+            for (int x = tid; x < words; x += OT) bits[x] = 0u;
+            __syncthreads();
+            for (uint32_t t = a + tid; t < b; t += OT) {
+                const uint32_t x = place_of(K[t]);
+                atomicOr(&bits[x >> 5], 1u << (x & 31u));
+            }
+            __syncthreads();
+            // ones before each thread's share of the words
+            uint32_t ones = 0u;
+            for (int x = tid * share; x < min((tid + 1) * share, words); ++x) ones += (uint32_t)__popc(bits[x]);
+            const uint32_t upto = wave_incl_scan(ones);
+            if (lane == 63) s_wave[w] = upto;
+            __syncthreads();
+            uint32_t first = upto - ones;
+            for (int k = 0; k < w; ++k) first += s_wave[k];
+            s_ones[tid] = first;
+            __syncthreads();
+            auto before = [&](uint32_t x) {
+                const int word = (int)(x >> 5);
+                if (word >= words) return b - a;
+                uint32_t r = s_ones[word / share];
+                for (int y = word / share * share; y < word; ++y) r += (uint32_t)__popc(bits[y]);
+                return r + (uint32_t)__popc(bits[word] & ((1u << (x & 31u)) - 1u));
+            };
+            for (uint32_t t = a + tid; t < b; t += OT)
+                put(t, c, before(place_of(K[t])), slabs ? before((uint32_t)n) : 0u, slabs ? before(2u * (uint32_t)n) : 0u,
+                    slabs ? before(3u * (uint32_t)n) : 0u);
+            __syncthreads();
+        }
+    };
+    if (count <= (uint32_t)kOneList) order(ordE, ordK, true);
+    else order(tmpE + base, tmpK + base, false);
+    __syncthreads();
+    for (int c = tid; c < own; c += OT) cs[c + lo] = table[c];
+    if (hi == m && tid == 0) cs[m] = (uint32_t)n;
 }
 
 inline int cblocks(int64_t n) { return (int)((n + CT - 1) / CT); }
 
 }  // namespace
 
-bool cell_sort_global(const sph_ctx* c) { return !(c->sc.cs_cells <= kLdsSortCells && c->n <= kLdsSortMax); }
+bool cell_sort_one(const sph_ctx* c) {
+    return c->n <= kOneSort && c->sc.cs_cells <= kOneGroups * kOneCells;
+}
 
 int64_t cell_scan_tiles(int64_t cells) { return (cells + CTILE - 1) / CTILE; }
 
@@ -373,18 +545,15 @@ hipError_t launch_cell_sort(sph_ctx* c, bool gather, hipStream_t s, bool counted
     uint32_t* tmp = b.valS[0];
     const int tiles = (int)cell_scan_tiles(m);
     const SlabTable T = slab_table(c->sc);
-    if (!cell_sort_global(c)) {
-        cell_sort_lds_kernel<<<1, LT, 0, s>>>(n, m, b.keyI, rank, b.cs, tmp, T);
-        if (n > 0) {
-            if (gather)
-                cell_order_kernel<true><<<cblocks(n), CT, 0, s>>>(n, T, tmp, b.keyI, b.cs, b.keyS[1], b.valS[1],
-                                                                   b.posB, b.velB, b.pidB, b.posA, b.velA, b.pidA);
-            else
-                cell_order_kernel<false><<<cblocks(n), CT, 0, s>>>(n, T, tmp, b.keyI, b.cs, b.keyS[1], b.valS[1],
-                                                                    nullptr, nullptr, b.pidB, nullptr, nullptr, nullptr);
-        }
-        c->sorted_keys = b.keyS[1];
-        c->sorted_vals = b.valS[1];
+    c->sorted_keys = b.keyS[1];
+    c->sorted_vals = b.valS[1];
+    if (cell_sort_one(c)) {
+        const int per = std::max(1, (m + kOneGroups - 1) / kOneGroups);
+        const int groups = std::max(1, (m + per - 1) / per);
+        const size_t lds = sizeof(uint32_t) * ((size_t)3 * per + 1 + 4 * kOneList + heavy_words(n, gather && T.shift > 0));
+        (gather ? cell_sort_one_kernel<true> : cell_sort_one_kernel<false>)<<<groups, OT, lds, s>>>(
+            n, m, per, T, b.keyI, b.pidB, b.cs, b.keyS[1], b.valS[1], b.posB, b.velB, b.posA, b.velA, b.pidA, tmp,
+            rank);
         return hipGetLastError();
     }
     const bool summed = counted && tile_sums_in_force(c);
@@ -410,8 +579,6 @@ hipError_t launch_cell_sort(sph_ctx* c, bool gather, hipStream_t s, bool counted
             cell_order_kernel<false><<<cblocks(n), CT, 0, s>>>(n, T, tmp, b.keyI, b.cs, b.keyS[1], b.valS[1], nullptr,
                                                                 nullptr, b.pidB, nullptr, nullptr, nullptr);
     }
-    c->sorted_keys = b.keyS[1];
-    c->sorted_vals = b.valS[1];
     return hipGetLastError();
 }
 

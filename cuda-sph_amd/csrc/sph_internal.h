@@ -229,10 +229,10 @@ hipError_t launch_upload_f32(sph_ctx* c, const float* x, const float* y, const f
 hipError_t launch_radix_sort_impl(sph_ctx* c, bool gather, hipStream_t s);
 // sph_cellsort.hip; also builds cs.  counted: the previous force pass counted the keys
 hipError_t launch_cell_sort(sph_ctx* c, bool gather, hipStream_t s, bool counted = false);
-// whether the counting sort runs on the global path (per-cell counts in cell_cnt), not in LDS
-bool cell_sort_global(const sph_ctx* c);
+// whether that sort runs in one launch (few particles)
+bool cell_sort_one(const sph_ctx* c);
 // whether the force pass can count the keys it writes for the next step's counting sort:
-// a plain (not batched) NAIVE step on the global sort path
+// a plain (not batched) NAIVE step whose sort takes several launches
 bool count_in_force(const sph_ctx* c);
 // lanes that share a particle of a plain context with one lane per particle (ordered sums)
 int ordered_lanes(const sph_ctx* c);

@@ -992,7 +992,7 @@ void launch_force_mode(sph_ctx* c, hipStream_t s, bool count) {
 }
 
 bool count_in_force(const sph_ctx* c) {
-    return c->cell_sort && c->inst.empty() && c->sc.formulation == SPH_FORM_NAIVE && cell_sort_global(c);
+    return c->cell_sort && c->inst.empty() && c->sc.formulation == SPH_FORM_NAIVE && !cell_sort_one(c);
 }
 
 bool tile_sums_in_force(const sph_ctx* c) { return count_in_force(c) && c->lanes == 1 && ordered_lanes(c) == 1; }
