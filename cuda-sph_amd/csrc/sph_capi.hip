@@ -225,10 +225,11 @@ int plan_instance(const sph_params_t& P, const sph_constants_t& K, sph::StepCons
 // left above the fields (up to 16) keep the cell's count where it fits.  The VOXEL
 // formulation keeps the reference's table.
 void plan_slabs(sph_ctx* c) {
-    constexpr int kField = 3;
+    constexpr int kField = sph::kSlabBits;
     int shift = 0, start_bits = 32, field = 0;
     if (c->sc.formulation == SPH_FORM_NAIVE) {
-        const int need = bit_length((uint64_t)(c->n > 0 ? c->n : 1));
+        // slab_field shifts the fields down to kSlabBits
+        const int need = std::max(kField, bit_length((uint64_t)(c->n > 0 ? c->n : 1)));
         for (int sh = c->whole_cells ? 0 : SPH_SLAB_SHIFT; sh > 0; --sh) {
             if (need + kField * ((1 << sh) - 1) <= 32) {
                 shift = sh;
@@ -247,6 +248,7 @@ void plan_slabs(sph_ctx* c) {
         S.count_pos = count_pos;
         S.count_bits = count_bits;
         S.start_mask = start_bits >= 32 ? ~0u : (1u << start_bits) - 1u;
+        S.field_mask = ((1u << (field * ((1 << shift) - 1))) - 1u) << kField;
     };
     apply(c->sc);
     for (auto& S : c->inst) apply(S);

@@ -99,8 +99,11 @@ __device__ __forceinline__ uint32_t sort_key(float x, float y, float z, const St
 // from it (0 for k = 0, and 0 when not known); see StepConsts::slab_shift.
 __device__ __forceinline__ uint32_t table_start(uint32_t w, const StepConsts& C) { return w & C.start_mask; }
 __device__ __forceinline__ uint32_t slab_field(uint32_t w, uint32_t k, const StepConsts& C) {
-    return __builtin_amdgcn_ubfe(w, (uint32_t)(C.start_bits + C.slab_bits * ((int)k - 1)),
-                                 k ? (uint32_t)C.slab_bits : 0u);
+    // the three fields with a zero field for slab 0 below them (start_bits is above slab_bits):
+    // no select for k = 0, and no 32-bit product (a quarter-rate instruction)
+    static_assert(kSlabBits == 3, "3 k from a shift and an add");
+    const uint32_t fields = (w >> (C.start_bits - kSlabBits)) & C.field_mask;
+    return __builtin_amdgcn_ubfe(fields, k + 2u * k, kSlabBits);
 }
 
 // bucket of a sort key in the cell table: -1 below the grid, n_cells above it

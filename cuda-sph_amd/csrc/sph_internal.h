@@ -124,9 +124,11 @@ struct StepConsts {
     int count_pos;
     int count_bits;
     uint32_t start_mask;  // the low start_bits bits
+    uint32_t field_mask;  // the bits of the offset fields once shifted down to kSlabBits
 };
 
 constexpr int kSlabKeyShift = 30;
+constexpr int kSlabBits = 3;  // StepConsts::slab_bits where cells are cut
 constexpr uint32_t kCellKeyMask = (1u << kSlabKeyShift) - 1u;
 // The counting sort's scan works in tiles of 2^kScanTileShift cells.  A tile's sum is kept
 // in kTileSumCopies places (cell_part: copy k of tile t at k * tiles + t, the sum is over the

@@ -180,11 +180,11 @@ constexpr uint32_t kOrderedTerms = 128;
 // is summed per lane, then across the group.  G holds the totals (particle count, cell
 // table length), C the particle's own instance; band is the particle's place in its
 // wavefront's LDS staging band
-// (unique in the workgroup), gbase its group's first lane in the wavefront.  FAR (L = 1): lists
-// beyond the int16 window too (kSeqList).  ORDERED (L > 1): the density is summed over the hits
+// (unique in the workgroup), gbase its group's first lane in the wavefront.  MASKED (L = 1): three
+// candidates at a time.  FAR (L = 1): lists beyond the int16 window too (kSeqList).  ORDERED (L > 1): the density is summed over the hits
 // in list order, as one lane sums it, to the same bits: the group keeps the hits' terms in terms
 // (kOrderedTerms words of LDS) and adds them up from there.
-template <int L, bool FAR = false, bool ORDERED = false>
+template <int L, bool FAR = false, bool ORDERED = false, bool MASKED = false>
 __device__ __forceinline__ void density_particle(const StepConsts& G, const StepConsts& C, int i, uint32_t l,
                                                  StageBand<L> band, uint32_t gbase, float4* pos, float4* vel,
                                                  const uint32_t* __restrict__ cs, float* __restrict__ rhoA,
@@ -217,10 +217,10 @@ __device__ __forceinline__ void density_particle(const StepConsts& G, const Step
     };
     // one candidate: a hit (r^2 <= h^2) adds (1 - r^2/h^2)^3 to the sum and is appended to the
     // list; CHECKED: the list may be full (staged slots, then HBM slots, then only counted)
-    auto visit = [&](float4 q, uint32_t k, auto checked) {
+    auto visit = [&](float4 q, uint32_t k, bool in_row, auto checked) {
         const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
         const float r2 = norm2(dx, dy, dz);
-        if (r2 <= C.h2) {
+        if (in_row && r2 <= C.h2) {
             const float t = 1.0f - r2 * C.inv_h2;
             acc += t * t * t;
             if constexpr (decltype(checked)::value) {
@@ -241,14 +241,23 @@ __device__ __forceinline__ void density_particle(const StepConsts& G, const Step
             auto walk = [&](auto checked) {
                 uint32_t off = k0 * 16u;
                 const uint32_t end = k1 * 16u;
-                for (; off + 16u * (kDensityUnroll - 1) < end; off += 16u * kDensityUnroll) {
-                    float4 q[kDensityUnroll];
+                if constexpr (MASKED) {  // three candidates at a time, those past the row's end masked out
+                    for (; off < end; off += 48u) {
+                        const float4 q[3] = {ld_f4(rpos, off), ld_f4(rpos, off + 16u), ld_f4(rpos, off + 32u)};
 #pragma unroll
-                    for (int u = 0; u < kDensityUnroll; ++u) q[u] = ld_f4(rpos, off + 16u * u);
+                        for (int u = 0; u < 3; ++u)
+                            visit(q[u], (off >> 4) + (uint32_t)u, u == 0 || off + 16u * u < end, checked);
+                    }
+                } else {
+                    for (; off + 16u * (kDensityUnroll - 1) < end; off += 16u * kDensityUnroll) {
+                        float4 q[kDensityUnroll];
 #pragma unroll
-                    for (int u = 0; u < kDensityUnroll; ++u) visit(q[u], (off >> 4) + (uint32_t)u, checked);
+                        for (int u = 0; u < kDensityUnroll; ++u) q[u] = ld_f4(rpos, off + 16u * u);
+#pragma unroll
+                        for (int u = 0; u < kDensityUnroll; ++u) visit(q[u], (off >> 4) + (uint32_t)u, true, checked);
+                    }
+                    for (; off < end; off += 16u) visit(ld_f4(rpos, off), off >> 4, true, checked);
                 }
-                for (; off < end; off += 16u) visit(ld_f4(rpos, off), off >> 4, checked);
             };
             // while every active lane's list has room in LDS for all of the row's candidates, the
             // row's hits need no capacity checks (a wave-uniform choice)
@@ -333,7 +342,7 @@ __device__ __forceinline__ void density_particle(const StepConsts& G, const Step
 
 // Plain step: L lanes per particle (1, 2, 4, 8, 16, 32 or 64), particle gt / L.  Groups are aligned,
 // so a whole group leaves together at the end of the range.
-template <int L, bool FAR = false, bool ORDERED = false>
+template <int L, bool FAR = false, bool ORDERED = false, bool MASKED = false>
 __global__ __launch_bounds__(kDensityThreads) void naive_density_kernel(StepConsts G, float4* pos, float4* vel,
                                                                          const uint32_t* __restrict__ cs,
                                                                          float* __restrict__ rhoA,
@@ -347,7 +356,7 @@ __global__ __launch_bounds__(kDensityThreads) void naive_density_kernel(StepCons
     const uint32_t lane = threadIdx.x & 63u;
     const StageBand<L> band{s_stage[threadIdx.x >> 6], lane / L};
     __shared__ __align__(16) float s_terms[ORDERED ? kDensityThreads / L : 1][ORDERED ? kOrderedTerms : 1];
-    density_particle<L, FAR, ORDERED>(G, G, i, gt & (L - 1), band, lane & ~(uint32_t)(L - 1), pos, vel, cs, rhoA, nl, nn,
+    density_particle<L, FAR, ORDERED, MASKED>(G, G, i, gt & (L - 1), band, lane & ~(uint32_t)(L - 1), pos, vel, cs, rhoA, nl, nn,
                                       s_terms[ORDERED ? threadIdx.x / L : 0]);
 }
 
@@ -831,6 +840,14 @@ constexpr int kDiagBlocks = 512;
 // particle does (1.36 against 1.92 ms per step).
 constexpr int64_t kFarParticles = int64_t(1) << 20;
 
+// Up to this many particles the one-lane density pass takes a row's candidates three at a time and
+// masks those past its end: few wavefronts share a SIMD then and wait on each other's loads
+// little, so a wait less per row counts.  With more of them the loads that are masked out cost
+// more (the pass is bound by the L1 data path).  us per launch, pairs and a remainder / threes:
+// dam break of 119,621 particles 40.7 / 36.2, 307,200 52.0 / 51.5, 516,096 71.3 / 71.8, pipe of
+// 262,144 63.1 / 57.6, 400,000 89.8 / 96.1.
+constexpr int64_t kMaskedParticles = 307200;
+
 // Lanes that share a particle in the density and force passes of a plain context with one lane
 // per particle, summing in its order: one lane leaves the card idle on few particles.  us per
 // launch, density / force, with one lane, 8 and 16 (h for about 30 neighbours in the box, 105
@@ -885,11 +902,11 @@ hipError_t launch_rekey(sph_ctx* c, hipStream_t s) {
     return hipGetLastError();
 }
 
-template <int L, bool FAR = false, bool ORDERED = false>
+template <int L, bool FAR = false, bool ORDERED = false, bool MASKED = false>
 void launch_density_lanes(sph_ctx* c, hipStream_t s) {
     const int bs = c->density_block;
     const Buffers& b = c->b;
-    naive_density_kernel<L, FAR, ORDERED><<<blocks_for(c->n * L, bs), bs, 0, s>>>(c->sc, b.posA, b.velA, b.cs, b.rhoA, b.nl, b.nn);
+    naive_density_kernel<L, FAR, ORDERED, MASKED><<<blocks_for(c->n * L, bs), bs, 0, s>>>(c->sc, b.posA, b.velA, b.cs, b.rhoA, b.nl, b.nn);
 }
 
 hipError_t launch_density(sph_ctx* c, hipStream_t s) {
@@ -919,7 +936,8 @@ hipError_t launch_density(sph_ctx* c, hipStream_t s) {
                 case 16: launch_density_lanes<16, false, true>(c, s); break;
                 case 8: launch_density_lanes<8, false, true>(c, s); break;
                 default:
-                    if (c->n > kFarParticles) launch_density_lanes<1, true>(c, s);
+                    if (c->n <= kMaskedParticles) launch_density_lanes<1, false, false, true>(c, s);
+                    else if (c->n > kFarParticles) launch_density_lanes<1, true>(c, s);
                     else launch_density_lanes<1>(c, s);
             }
             break;

@@ -26,3 +26,10 @@ def test_ordered_groups_sum_as_one_lane(gpu, n, mean):
     got = NaiveSPHStrategy(w.params, constants=w.constants, device=gpu).advance(state, 3)
     for f in ("position", "velocity", "density"):
         assert np.array_equal(getattr(got, f), getattr(want, f)), f
+
+
+# up to 307,200 particles one lane takes its candidates in threes, past that in pairs, in a batch
+# in pairs; 60 neighbours fill the staged list slots, 130 all of them
+@pytest.mark.parametrize("n,mean", [(98305, 60), (110003, 130), (307200, 30), (307201, 30)])
+def test_threes_and_pairs_sum_alike(gpu, n, mean):
+    test_ordered_groups_sum_as_one_lane(gpu, n, mean)
