@@ -111,13 +111,6 @@ __device__ __forceinline__ void walk_neighbours_lanes(const StepConsts& C, int i
     }
 }
 
-template <int L>
-__device__ __forceinline__ float group_sum(float v) {
-#pragma unroll
-    for (int o = 1; o < L; o <<= 1) v += __shfl_xor(v, o);
-    return v;
-}
-
 __device__ __forceinline__ float comp(const Vec3& a, int d) { return d == 0 ? a.x : (d == 1 ? a.y : a.z); }
 __device__ __forceinline__ float comp(const float4& a, int d) { return d == 0 ? a.x : (d == 1 ? a.y : a.z); }
 

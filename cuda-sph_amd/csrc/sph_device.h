@@ -54,6 +54,37 @@ __device__ __forceinline__ const StepConsts& inst_consts(const StepConsts& G, in
 }
 
 
+// The value of lane (own lane) ^ O for O = 1, 2, 16 and, where every aligned group of O lanes holds
+// one value, O = 4 and 8 (by mirroring: lane 7 - i and 15 - i of the row): as the steps of a sum
+// over a group these need no LDS access up to 8, against a ds_bpermute and its address each.
+// The sums come out as those of __shfl_xor, bit for bit.
+template <int O>
+__device__ __forceinline__ uint32_t lane_xor(uint32_t v) {
+    if constexpr (O == 1) return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xb1, 0xf, 0xf, true);   // quad_perm 1 0 3 2
+    else if constexpr (O == 2) return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4e, 0xf, 0xf, true);  // 2 3 0 1
+    else if constexpr (O == 4) return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xf, 0xf, true);  // row_half_mirror
+    else if constexpr (O == 8) return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xf, 0xf, true);  // row_mirror
+    else if constexpr (O == 16) return (uint32_t)__builtin_amdgcn_ds_swizzle((int)v, 0x401f);  // xor 16 within 32
+    else return (uint32_t)__shfl_xor((int)v, O);
+}
+// Combination of one value per lane over each group of L lanes, in all of them.
+template <int L, typename F>
+__device__ __forceinline__ uint32_t group_fold(uint32_t v, F&& f) {
+    if constexpr (L > 1) v = f(v, lane_xor<1>(v));
+    if constexpr (L > 2) v = f(v, lane_xor<2>(v));
+    if constexpr (L > 4) v = f(v, lane_xor<4>(v));
+    if constexpr (L > 8) v = f(v, lane_xor<8>(v));
+    if constexpr (L > 16) v = f(v, lane_xor<16>(v));
+    if constexpr (L > 32) v = f(v, lane_xor<32>(v));
+    return v;
+}
+template <int L>
+__device__ __forceinline__ float group_sum(float v) {
+    return __uint_as_float(group_fold<L>(__float_as_uint(v), [](uint32_t a, uint32_t b) {
+        return __float_as_uint(__uint_as_float(a) + __uint_as_float(b));
+    }));
+}
+
 // Raw buffer loads with 32-bit byte offsets: no 64-bit address arithmetic per access, and
 // an offset past num_records reads zero instead of faulting.  Word 3 of the descriptor is
 // the gfx9 value for untyped 32-bit-element buffers.
@@ -762,15 +793,12 @@ __device__ __forceinline__ PairSums naive_pair_sums_lanes(const StepConsts& C, i
                 },
                 tail);
         }
-#pragma unroll
-        for (int o = 1; o < L; o <<= 1) {
-            S.ax += __shfl_xor(S.ax, o);
-            S.ay += __shfl_xor(S.ay, o);
-            S.az += __shfl_xor(S.az, o);
-            S.bx += __shfl_xor(S.bx, o);
-            S.by += __shfl_xor(S.by, o);
-            S.bz += __shfl_xor(S.bz, o);
-        }
+        S.ax = group_sum<L>(S.ax);
+        S.ay = group_sum<L>(S.ay);
+        S.az = group_sum<L>(S.az);
+        S.bx = group_sum<L>(S.bx);
+        S.by = group_sum<L>(S.by);
+        S.bz = group_sum<L>(S.bz);
         return S;
     }
 }

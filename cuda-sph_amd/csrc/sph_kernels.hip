@@ -310,16 +310,10 @@ __device__ __forceinline__ void density_particle(const StepConsts& G, const Step
                 kept += (uint32_t)__popcll(gm);
             });
         if (ORDERED) add_terms();
-#pragma unroll
-        for (int o = 1; o < L; o <<= 1) {
-            klo = min(klo, (uint32_t)__shfl_xor(klo, o));
-            khi = max(khi, (uint32_t)__shfl_xor(khi, o));
-        }
+        klo = group_fold<L>(klo, [](uint32_t a, uint32_t b) { return min(a, b); });
+        khi = group_fold<L>(khi, [](uint32_t a, uint32_t b) { return max(a, b); });
     }
-    if (!ORDERED) {
-#pragma unroll
-        for (int o = 1; o < L; o <<= 1) acc += __shfl_xor(acc, o);
-    }
+    if (!ORDERED) acc = group_sum<L>(acc);
     const uint32_t staged = cnt < kCap ? cnt : kCap;
     // the staged slots as 32-bit words (two slots each), the group's lanes taking turns
     uint32_t* words = reinterpret_cast<uint32_t*>(nl);
