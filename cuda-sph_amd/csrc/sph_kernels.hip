@@ -384,6 +384,11 @@ __device__ __forceinline__ BatchLane batch_lane(const StepConsts& G, uint32_t gt
     return r;
 }
 
+// TOP, 16 or 64, is the largest group that the kernel has code for: the path of 32 lanes over rows
+// laid end to end costs the others 4% where it stands beside them (64 boxes of 2,048 to 65,536
+// particles at up to 16 lanes, 4 steps: 5.98 ms, 5.74 without it).  A larger group than TOP, which
+// a graph captured before the lanes were set can meet, works with its first TOP lanes.
+template <int TOP>
 __global__ __launch_bounds__(kDensityThreads) void naive_density_batch_kernel(StepConsts G, float4* pos, float4* vel,
                                                                                const uint32_t* __restrict__ cs,
                                                                                float* __restrict__ rhoA,
@@ -404,8 +409,15 @@ __global__ __launch_bounds__(kDensityThreads) void naive_density_batch_kernel(St
         case 4: density_particle<4>(G, C, t.i, t.l, StageBand<4>{base, p}, gbase, pos, vel, cs, rhoA, nl, nn); break;
         case 8: density_particle<8>(G, C, t.i, t.l, StageBand<8>{base, p}, gbase, pos, vel, cs, rhoA, nl, nn); break;
         case 16: density_particle<16>(G, C, t.i, t.l, StageBand<16>{base, p}, gbase, pos, vel, cs, rhoA, nl, nn); break;
-        case 32: density_particle<32>(G, C, t.i, t.l, StageBand<32>{base, p}, gbase, pos, vel, cs, rhoA, nl, nn); break;
-        default: density_particle<64>(G, C, t.i, t.l, StageBand<64>{base, p}, gbase, pos, vel, cs, rhoA, nl, nn); break;
+        case 32:
+            if constexpr (TOP > 32) {
+                density_particle<32>(G, C, t.i, t.l, StageBand<32>{base, p}, gbase, pos, vel, cs, rhoA, nl, nn);
+                break;
+            }
+            [[fallthrough]];
+        default:
+            if (t.l < (uint32_t)TOP)
+                density_particle<TOP>(G, C, t.i, t.l, StageBand<TOP>{base, p}, gbase, pos, vel, cs, rhoA, nl, nn);
     }
 }
 
@@ -468,6 +480,7 @@ __global__ __launch_bounds__(256) void naive_force_kernel(
 }
 
 // Batched form of the force pass (box walls): the thread map of naive_density_batch_kernel.
+template <int TOP>
 __global__ __launch_bounds__(256) void naive_force_batch_kernel(
     StepConsts G, const float4* __restrict__ pos, const float4* __restrict__ vel, const uint32_t* __restrict__ pidA,
     const float* __restrict__ rhoA, const uint32_t* __restrict__ cs, const ListEntry* __restrict__ nl,
@@ -487,8 +500,14 @@ __global__ __launch_bounds__(256) void naive_force_batch_kernel(
         case 4: S = naive_pair_sums_lanes<4>(C, i, t.l, G.n, p, v, pos, vel, cs, nl, nn); break;
         case 8: S = naive_pair_sums_lanes<8>(C, i, t.l, G.n, p, v, pos, vel, cs, nl, nn); break;
         case 16: S = naive_pair_sums_lanes<16>(C, i, t.l, G.n, p, v, pos, vel, cs, nl, nn); break;
-        case 32: S = naive_pair_sums_lanes<32>(C, i, t.l, G.n, p, v, pos, vel, cs, nl, nn); break;
-        default: S = naive_pair_sums_lanes<64>(C, i, t.l, G.n, p, v, pos, vel, cs, nl, nn); break;
+        case 32:
+            if constexpr (TOP > 32) {
+                S = naive_pair_sums_lanes<32>(C, i, t.l, G.n, p, v, pos, vel, cs, nl, nn);
+                break;
+            }
+            [[fallthrough]];
+        default:
+            if (t.l < (uint32_t)TOP) S = naive_pair_sums_lanes<TOP>(C, i, t.l, G.n, p, v, pos, vel, cs, nl, nn);
     }
     if (t.l != 0) return;
     const float ps = 0.5f * C.mass * C.grad_c;
@@ -903,6 +922,14 @@ void launch_density_lanes(sph_ctx* c, hipStream_t s) {
     naive_density_kernel<L, FAR, ORDERED, MASKED><<<blocks_for(c->n * L, bs), bs, 0, s>>>(c->sc, b.posA, b.velA, b.cs, b.rhoA, b.nl, b.nn);
 }
 
+// Most lanes of an instance: up to 16, the batch's passes leave out what 32 and 64 lanes need
+// (naive_density_batch_kernel).
+int batch_top_lanes(const sph_ctx* c) {
+    int top = 1;
+    for (const StepConsts& S : c->inst) top = max(top, S.lanes);
+    return top;
+}
+
 hipError_t launch_density(sph_ctx* c, hipStream_t s) {
     if (c->n == 0) return hipGetLastError();
     const int bs = c->density_block;
@@ -914,7 +941,8 @@ hipError_t launch_density(sph_ctx* c, hipStream_t s) {
     }
     if (!c->inst.empty()) {
         const Buffers& b = c->b;
-        naive_density_batch_kernel<<<blocks_for(c->sc.tfirst, bs), bs, 0, s>>>(c->sc, b.posA, b.velA, b.cs, b.rhoA,
+        const auto kernel = batch_top_lanes(c) > 16 ? naive_density_batch_kernel<64> : naive_density_batch_kernel<16>;
+        kernel<<<blocks_for(c->sc.tfirst, bs), bs, 0, s>>>(c->sc, b.posA, b.velA, b.cs, b.rhoA,
                                                                               b.nl, b.nn);
         return hipGetLastError();
     }
@@ -963,7 +991,8 @@ void launch_force_mode(sph_ctx* c, hipStream_t s, bool count) {
         return;
     }
     if (!c->inst.empty()) {  // batched instances have box walls
-        naive_force_batch_kernel<<<blocks_for(c->sc.tfirst, bs), bs, 0, s>>>(
+        const auto kernel = batch_top_lanes(c) > 16 ? naive_force_batch_kernel<64> : naive_force_batch_kernel<16>;
+        kernel<<<blocks_for(c->sc.tfirst, bs), bs, 0, s>>>(
             c->sc, c->b.posA, c->b.velA, c->b.pidA, c->b.rhoA, c->b.cs, c->b.nl, c->b.nn, c->b.posB, c->b.velB,
             c->b.pidB, c->b.keyI, c->b.valI, dP, dV, dF, c->b.flags);
         return;
