@@ -355,6 +355,44 @@ __device__ __forceinline__ void for_each_candidate(float px, float py, float pz,
     });
 }
 
+// The rows [k0, k1) of a group's L lanes (k0 <= k1) laid end to end in lane order: the row of lane l
+// has the places [start, start + k1 - k0) of `total`, and window() gives lane l the candidate at
+// place `at` + l, for at = 0, L, ... in turn with one `seen` (past the last place: anything).
+template <int L>
+struct RowWindows {
+    static_assert(L == 32, "starts are bits of one word");
+    uint32_t total, start, l;
+    uint32_t shift;  // of the l-th row that is not empty: k0 less start
+    int gbase;
+    bool any;
+    __device__ __forceinline__ RowWindows(uint32_t k0, uint32_t k1, uint32_t lane, int base) : l(lane), gbase(base) {
+        const uint32_t len = k1 - k0;
+        any = len != 0u;
+        uint32_t sum = len;
+#pragma unroll
+        for (int o = 1; o < L; o <<= 1) {
+            const uint32_t y = __shfl_up(sum, o, L);
+            if ((int)l >= o) sum += y;
+        }
+        total = __shfl(sum, L - 1, L);
+        start = sum - len;
+        // the rows that are not empty to the first lanes
+        const uint32_t full = (uint32_t)(__ballot(any) >> gbase);
+        const uint32_t before = (uint32_t)__popc(full & ((1u << l) - 1u));
+        const uint32_t to = any ? before : (uint32_t)__popc(full) + l - before;
+        shift = (uint32_t)__builtin_amdgcn_ds_permute((gbase + (int)to) * 4, (int)(k0 - start));
+    }
+    // seen: rows that start before the window
+    __device__ __forceinline__ uint32_t window(uint32_t& seen, uint32_t at) const {
+        const uint32_t rel = start - at;
+        const uint32_t starts = group_fold<L>(any && rel < (uint32_t)L ? 1u << rel : 0u,
+                                              [](uint32_t x, uint32_t y) { return x | y; });
+        const uint32_t row = seen + (uint32_t)__popc(starts & ((2u << l) - 1u)) - 1u;
+        seen += (uint32_t)__popc(starts);
+        return (uint32_t)__shfl((int)shift, gbase + (int)row) + at + l;
+    }
+};
+
 // for_each_row for a group of L lanes sharing one particle (groups aligned in the
 // wavefront, l the lane's index in its group): the particle's (cy, cz) pairs are numbered
 // t = 0, 1, ... in for_each_row's order, lane l works out the rows of pairs l, l + L, ...
@@ -393,41 +431,19 @@ __device__ __forceinline__ void for_each_batch(float px, float py, float pz, con
         }
         uint64_t left = (__ballot(a0 < a1) >> gbase) & group;  // the rows that hold candidates
         if constexpr (L == 32) {
-            // row of candidates [a0, a1) at places [start, start + len)
-            const uint32_t len = a1 - a0;
-            uint32_t start = len;
-#pragma unroll
-            for (int o = 1; o < L; o <<= 1) {
-                const uint32_t y = __shfl_up(start, o, L);
-                if ((int)l >= o) start += y;
-            }
-            const uint32_t total = __shfl(start, L - 1, L);
-            start -= len;
-            // candidate less place of the rows that hold any, one after the other in the group's lanes
-            const uint32_t before = (uint32_t)__popcll(left & ((1ull << l) - 1ull));
-            const uint32_t to = len ? before : (uint32_t)__popcll(left) + l - before;
-            const uint32_t shift = (uint32_t)__builtin_amdgcn_ds_permute((gbase + (int)to) * 4, (int)(a0 - start));
-            uint32_t begun = 0u;  // rows that start before the window
-            // the candidate at place `at` + l: its row is the last that starts up to there
-            auto window = [&](uint32_t at) {
-                const uint32_t rel = start - at;
-                const uint32_t starts = group_fold<L>(len && rel < (uint32_t)L ? 1u << rel : 0u,
-                                                      [](uint32_t x, uint32_t y) { return x | y; });
-                const uint32_t r = begun + (uint32_t)__popc(starts & ((2u << l) - 1u)) - 1u;
-                begun += (uint32_t)__popc(starts);
-                return (uint32_t)__shfl((int)shift, gbase + (int)r) + at + l;
-            };
-            if (total == 0u) continue;
-            uint32_t k = window(0u);
+            const RowWindows<L> line(a0, a1, l, gbase);
+            if (line.total == 0u) continue;
+            uint32_t seen = 0u;
+            uint32_t k = line.window(seen, 0u);
             float4 q = ld_f4(rpos, k * 16u);
-            for (uint32_t at = 0u; at < total; at += L) {
+            for (uint32_t at = 0u; at < line.total; at += L) {
                 const uint32_t kc = k;
                 const float4 qc = q;
-                if (at + L < total) {
-                    k = window(at + L);
+                if (at + L < line.total) {
+                    k = line.window(seen, at + L);
                     q = ld_f4(rpos, k * 16u);
                 }
-                f(kc, qc, at + l < total);
+                f(kc, qc, at + l < line.total);
             }
             continue;
         }
