@@ -7,10 +7,11 @@
 // laid out in particle-id order, so a stable sort on the key alone reproduces that order.
 //
 // Each pass sorts on up to 8 key bits with three launches:
-//   upsweep   one workgroup per 2048-key tile counts digits in LDS (one histogram per
-//             wavefront to spread LDS atomics) and writes counts digit-major;
+//   upsweep   one workgroup per tile of 512, 1024 or 2048 keys counts digits in LDS (one
+//             histogram per wavefront to spread LDS atomics) and writes counts digit-major;
 //   scan      one workgroup per digit turns the counts of that digit into exclusive
-//             tile offsets and a digit total;
+//             tile offsets and a digit total (few tiles: the upsweep writes tile-major and
+//             each workgroup of the downsweep adds the counts up itself, without this launch);
 //   downsweep each tile ranks its keys stably with wave64 ballots (the lanes holding the
 //             same digit are found with one ballot per digit bit), places them in LDS in
 //             digit order and writes each digit run contiguously.  On the last pass it can
@@ -25,9 +26,15 @@ constexpr int RB = 8;
 constexpr int RADIX = 1 << RB;   // 256 digits
 constexpr int ST = 256;          // threads per workgroup, 4 wavefronts
 constexpr int WAVES = ST / 64;
-constexpr int SI = 8;            // keys per thread
-constexpr int TILE = ST * SI;    // 2048 keys per tile
-static_assert(RADIX == ST, "one digit per thread in the per-digit phases");
+
+// Keys per thread (a tile is 256 times as many): a pass over few keys is a chain of waits, which more
+// and smaller tiles shorten, until their counts and short runs of equal digits cost more than
+// that.  Up to kFewTiles tiles the downsweep adds all counts up.  us per sort with the gather
+// (dam break, 2 / 4 / 8 keys with the scan): 55,296 particles 45 / 52 / 66, 131,072 51 / 55 / 70,
+// 262,144 60 / 59 / 71, 524,288 - / 70 / 75, 1,048,576 - / 105 / 102; 2 keys without / 8 with the
+// scan: 4,096 33 / 64, 24,576 42 / 65, 49,152 51 / 66.
+constexpr int kFewTiles = 96;
+int keys_per_thread(int64_t n) { return n <= 196608 ? 2 : n <= 786432 ? 4 : 8; }
 
 // Exclusive scan of one value per thread across the 256-thread workgroup.
 __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* lds_wave, uint32_t* total) {
@@ -52,6 +59,7 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* lds_wa
     return woff + x - v;
 }
 
+template <int SI, bool FEW>
 __global__ __launch_bounds__(ST) void radix_upsweep(const uint32_t* __restrict__ keys, int n, int shift,
                                                      uint32_t mask, uint32_t* __restrict__ hist, int ntiles,
                                                      uint32_t* __restrict__ clear_flag) {
@@ -62,7 +70,7 @@ __global__ __launch_bounds__(ST) void radix_upsweep(const uint32_t* __restrict__
     for (int i = threadIdx.x; i < WAVES * RADIX; i += ST) (&h[0][0])[i] = 0;
     __syncthreads();
     const int w = threadIdx.x >> 6;
-    const int64_t base = (int64_t)blockIdx.x * TILE;
+    const int64_t base = (int64_t)blockIdx.x * (ST * SI);
 #pragma unroll
     for (int k = 0; k < SI; ++k) {
         int64_t idx = base + k * ST + threadIdx.x;
@@ -73,7 +81,7 @@ __global__ __launch_bounds__(ST) void radix_upsweep(const uint32_t* __restrict__
     uint32_t s = 0;
 #pragma unroll
     for (int i = 0; i < WAVES; ++i) s += h[i][d];
-    hist[(int64_t)d * ntiles + blockIdx.x] = s;
+    hist[FEW ? (int64_t)blockIdx.x * RADIX + d : (int64_t)d * ntiles + blockIdx.x] = s;
 }
 
 __global__ __launch_bounds__(ST) void radix_scan_digits(uint32_t* __restrict__ hist, int ntiles,
@@ -95,7 +103,7 @@ __global__ __launch_bounds__(ST) void radix_scan_digits(uint32_t* __restrict__ h
 // GATHER (the last pass of the fused step): also gathers the state into cell order and, for
 // the VOXEL formulation (C.formulation), reports a position outside the voxel grid in
 // flags[kFlagOutOfGrid].
-template <bool GATHER>
+template <int SI, bool FEW, bool GATHER>
 __global__ __launch_bounds__(ST) void radix_downsweep(const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
                                                        uint32_t* __restrict__ kout, uint32_t* __restrict__ vout, int n,
                                                        int shift, int bits, const uint32_t* __restrict__ hist,
@@ -104,6 +112,7 @@ __global__ __launch_bounds__(ST) void radix_downsweep(const uint32_t* __restrict
                                                        const uint32_t* __restrict__ pidB, float4* __restrict__ posA,
                                                        float4* __restrict__ velA, uint32_t* __restrict__ pidA,
                                                        StepConsts C, uint32_t* __restrict__ flags) {
+    constexpr int TILE = ST * SI;
     __shared__ uint32_t s_keys[TILE];
     __shared__ uint32_t s_vals[TILE];
     __shared__ uint32_t s_whist[WAVES][RADIX];
@@ -117,9 +126,21 @@ __global__ __launch_bounds__(ST) void radix_downsweep(const uint32_t* __restrict
 
     for (int i = tid; i < WAVES * RADIX; i += ST) (&s_whist[0][0])[i] = 0;
     {
+        uint32_t all = 0, before = 0;
+        if constexpr (FEW) {
+#pragma unroll 8
+            for (int t = 0; t < ntiles; ++t) {
+                const uint32_t v = hist[t * RADIX + tid];
+                all += v;
+                before += t < (int)blockIdx.x ? v : 0u;
+            }
+        } else {
+            all = digit_total[tid];
+            before = hist[(int64_t)tid * ntiles + blockIdx.x];
+        }
         uint32_t tot;
-        uint32_t ex = block_excl_scan(digit_total[tid], s_lw, &tot);  // synchronises: s_whist zeroed
-        s_gbase[tid] = ex + hist[(int64_t)tid * ntiles + blockIdx.x];
+        uint32_t ex = block_excl_scan(all, s_lw, &tot);  // synchronises: s_whist zeroed
+        s_gbase[tid] = ex + before;
     }
 
     uint32_t key[SI], val[SI], rank[SI];
@@ -177,35 +198,76 @@ __global__ __launch_bounds__(ST) void radix_downsweep(const uint32_t* __restrict
     }
     __syncthreads();
     const int tile_n = (int)((n - base) < TILE ? (n - base) : TILE);
-    for (int i = tid; i < tile_n; i += ST) {
-        const uint32_t kk = s_keys[i];
-        const uint32_t vv = s_vals[i];
-        const uint32_t d = (kk >> shift) & mask;
-        const uint32_t g = s_gbase[d] + (uint32_t)i - s_tstart[d];
-        kout[g] = kk;
-        vout[g] = vv;
-        if (GATHER) {
-            const float4 p = posB[vv];
-            posA[g] = p;
-            velA[g] = velB[vv];
-            pidA[g] = pidB[vv];
-            if (C.formulation == SPH_FORM_VOXEL && outside_voxel_grid(p.x, p.y, p.z, C)) flags[kFlagOutOfGrid] = 1u;
+    // up to four keys' gathers in flight
+    constexpr int GI = SI < 4 ? SI : 4;
+    for (int i0 = tid; i0 < tile_n; i0 += ST * GI) {
+        uint32_t vv[GI], g[GI];
+#pragma unroll
+        for (int u = 0; u < GI; ++u) {
+            const int i = min(i0 + u * ST, tile_n - 1);
+            const uint32_t kk = s_keys[i];
+            const uint32_t d = (kk >> shift) & mask;
+            vv[u] = s_vals[i];
+            g[u] = s_gbase[d] + (uint32_t)i - s_tstart[d];
+            if (i0 + u * ST < tile_n) {
+                kout[g[u]] = kk;
+                vout[g[u]] = vv[u];
+            }
+        }
+        if constexpr (GATHER) {
+            float4 p[GI], v[GI];
+            uint32_t id[GI];
+#pragma unroll
+            for (int u = 0; u < GI; ++u) {
+                p[u] = posB[vv[u]];
+                v[u] = velB[vv[u]];
+                id[u] = pidB[vv[u]];
+            }
+#pragma unroll
+            for (int u = 0; u < GI; ++u) {
+                if (i0 + u * ST >= tile_n) break;
+                posA[g[u]] = p[u];
+                velA[g[u]] = v[u];
+                pidA[g[u]] = id[u];
+                if (C.formulation == SPH_FORM_VOXEL && outside_voxel_grid(p[u].x, p[u].y, p[u].z, C))
+                    flags[kFlagOutOfGrid] = 1u;
+            }
         }
     }
 }
 
+// One pass over the tiles.
+template <int SI, bool FEW>
+void launch_radix_pass(sph_ctx* c, int p, bool gather, const uint32_t* kin, const uint32_t* vin, uint32_t* kout,
+                       uint32_t* vout, hipStream_t s) {
+    const int n = (int)c->n, T = c->num_tiles, shift = c->pass_shift[p], bits = c->pass_bits[p];
+    const Buffers& b = c->b;
+    radix_upsweep<SI, FEW><<<T, ST, 0, s>>>(kin, n, shift, (1u << bits) - 1u, b.tile_hist, T,
+                                           p == 0 ? b.flags + kFlagOutOfGrid : nullptr);
+    if (!FEW) radix_scan_digits<<<RADIX, ST, 0, s>>>(b.tile_hist, T, b.digit_total);
+    if (gather)
+        radix_downsweep<SI, FEW, true><<<T, ST, 0, s>>>(kin, vin, kout, vout, n, shift, bits, b.tile_hist,
+                                                       b.digit_total, T, b.posB, b.velB, b.pidB, b.posA, b.velA,
+                                                       b.pidA, c->sc, b.flags);
+    else
+        radix_downsweep<SI, FEW, false><<<T, ST, 0, s>>>(kin, vin, kout, vout, n, shift, bits, b.tile_hist,
+                                                        b.digit_total, T, nullptr, nullptr, nullptr, nullptr, nullptr,
+                                                        nullptr, c->sc, nullptr);
+}
+
 }  // namespace
 
-int radix_num_tiles(int64_t n) { return (int)((n + TILE - 1) / TILE); }
+int radix_num_tiles(int64_t n) {
+    const int64_t tile = (int64_t)ST * keys_per_thread(n);
+    return (int)((n + tile - 1) / tile);
+}
 
 // Sorts (keyI, valI) into the radix ping-pong buffers.  When gather is set the last pass
 // also writes posA/velA in sorted order; returns through c->sorted_keys/sorted_vals.
 hipError_t launch_radix_sort_impl(sph_ctx* c, bool gather, hipStream_t s) {
-    const int n = (int)c->n;
-    const int T = c->num_tiles;
     const uint32_t* kin = c->b.keyI;
     const uint32_t* vin = c->b.valI;
-    if (n == 0) {
+    if (c->n == 0) {
         c->sorted_keys = c->b.keyI;
         c->sorted_vals = c->b.valI;
         return hipGetLastError();
@@ -213,19 +275,14 @@ hipError_t launch_radix_sort_impl(sph_ctx* c, bool gather, hipStream_t s) {
     for (int p = 0; p < c->passes; ++p) {
         uint32_t* kout = c->b.keyS[p & 1];
         uint32_t* vout = c->b.valS[p & 1];
-        const int shift = c->pass_shift[p], bits = c->pass_bits[p];
-        const uint32_t mask = (1u << bits) - 1u;
-        radix_upsweep<<<T, ST, 0, s>>>(kin, n, shift, mask, c->b.tile_hist, T,
-                                         p == 0 ? c->b.flags + kFlagOutOfGrid : nullptr);
-        radix_scan_digits<<<RADIX, ST, 0, s>>>(c->b.tile_hist, T, c->b.digit_total);
-        if (gather && p == c->passes - 1)
-            radix_downsweep<true><<<T, ST, 0, s>>>(kin, vin, kout, vout, n, shift, bits, c->b.tile_hist,
-                                                    c->b.digit_total, T, c->b.posB, c->b.velB, c->b.pidB, c->b.posA,
-                                                    c->b.velA, c->b.pidA, c->sc, c->b.flags);
-        else
-            radix_downsweep<false><<<T, ST, 0, s>>>(kin, vin, kout, vout, n, shift, bits, c->b.tile_hist,
-                                                     c->b.digit_total, T, nullptr, nullptr, nullptr, nullptr, nullptr,
-                                                     nullptr, c->sc, nullptr);
+        const bool last = gather && p == c->passes - 1;
+        const bool few = c->num_tiles <= kFewTiles;
+        const int keys = keys_per_thread(c->n);
+        const auto pass = few         ? launch_radix_pass<2, true>
+                          : keys == 2 ? launch_radix_pass<2, false>
+                          : keys == 4 ? launch_radix_pass<4, false>
+                                      : launch_radix_pass<8, false>;
+        pass(c, p, last, kin, vin, kout, vout, s);
         kin = kout;
         vin = vout;
     }
