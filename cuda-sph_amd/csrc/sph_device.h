@@ -474,6 +474,100 @@ __device__ __forceinline__ void for_each_batch(float px, float py, float pz, con
     }
 }
 
+__device__ __forceinline__ float lane_of(float v, int lane) {
+    return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(v), lane));
+}
+
+// The candidate rows of the P particles that share a wavefront, 64 / P lanes each: a row runs from
+// the first to the last x slab that any of them reaches, so that each candidate is loaded once
+// and tested against all P.  The passes over dense particles are bound by the L1 data path (its
+// return path was busy 98% of the time with a load per pair).  ok: all P lie within about a cell of
+// each other and have at most 64 rows, one per lane.
+// With 16 lanes only, which dense instances get (us per step, density and force, before and
+// after: 51,680 particles of 2,626 neighbours 188 and 258 -> 137 and 211, 43,010 of 1,086 117 and
+// 161 -> 67 and 94, the 64-box batch 606 and 702 -> 508 and 578).
+// 8 lanes gained nothing (95,162 particles of 295 neighbours 115 and 154 -> 118 and 146, the force
+// kernel at 77 registers) and lost in the density pass with 4 (142 -> 165).
+template <int L>
+constexpr bool kSharesRows = L == 16;
+
+template <int P>
+struct SharedRows {
+    uint32_t k0 = 0u, k1 = 0u;  // the lane's row
+    bool ok;
+
+    __device__ __forceinline__ SharedRows(float4 p, const StepConsts& C, __amdgpu_buffer_rsrc_t rcs) {
+        const RowGrid R(p.x, p.y, p.z, C);
+        int ylo = R.ylo, yhi = R.yhi, zlo = R.zlo, zhi = R.zhi;
+        float xlo = R.fx, xhi = R.fx;
+#pragma unroll
+        for (int j = 0; j < P; ++j) {
+            const int at = j * (64 / P);
+            ylo = min(ylo, __builtin_amdgcn_readlane(R.ylo, at));
+            yhi = max(yhi, __builtin_amdgcn_readlane(R.yhi, at));
+            zlo = min(zlo, __builtin_amdgcn_readlane(R.zlo, at));
+            zhi = max(zhi, __builtin_amdgcn_readlane(R.zhi, at));
+            xlo = fminf(xlo, lane_of(R.fx, at));
+            xhi = fmaxf(xhi, lane_of(R.fx, at));
+        }
+        const int ny = yhi - ylo + 1, rows = ny * (zhi - zlo + 1);
+        const bool near = yhi - ylo <= R.yhi - R.ylo + 1 && zhi - zlo <= R.zhi - R.zlo + 1 &&
+                          xhi - xlo <= (float)(2 << C.slab_shift);
+        ok = __ballot(near && rows <= 64) == ~0ull;
+        if (!ok) return;
+        const int t = (int)(threadIdx.x & 63u);
+        const int cz = zlo + t / ny, cy = ylo + t % ny;
+        uint32_t q0 = 0xffffffffu, q1 = 0u;
+#pragma unroll
+        for (int j = 0; j < P; ++j) {
+            const int at = j * (64 / P);
+            const RowGrid one(lane_of(p.x, at), lane_of(p.y, at), lane_of(p.z, at), C);
+            uint32_t a, b;
+            if (t < rows && one.row(cy, one.rest_z(cz, C), C, a, b)) {
+                q0 = min(q0, a);
+                q1 = max(q1, b);
+            }
+        }
+        if (q0 < q1)
+            RowGrid::range(C.cell_off + C.dims[0] * (cy + C.dims[1] * cz), q0, q1, C,
+                           [&](int c) { return ld_u32(rcs, (uint32_t)c * 4u); }, k0, k1);
+    }
+
+    __device__ __forceinline__ uint32_t candidates() const { return group_fold<64>(k0 < k1 ? k1 - k0 : 0u, [](uint32_t a, uint32_t b) { return a + b; }); }
+
+    // f(k, ld(k), valid) by all 64 lanes together, lane l with the candidates k0 + l + 64 m of
+    // each row; the next batch is loaded before f gets this one's
+    template <typename LD, typename F>
+    __device__ __forceinline__ void walk(LD&& ld, F&& f) const {
+        const uint32_t l = threadIdx.x & 63u;
+        uint64_t left = __ballot(k0 < k1);
+        if (left == 0ull) return;
+        uint32_t b, e;
+        auto next_row = [&]() {
+            const int j = __ffsll((unsigned long long)left) - 1;
+            left &= left - 1ull;
+            b = (uint32_t)__builtin_amdgcn_readlane((int)k0, j);
+            e = (uint32_t)__builtin_amdgcn_readlane((int)k1, j);
+        };
+        next_row();
+        auto next = ld(min(b + l, e - 1u));
+        while (true) {
+            const uint32_t k = b + l;
+            const bool valid = k < e;
+            const auto now = next;
+            b += 64u;
+            bool more = true;
+            if (b >= e) {
+                more = left != 0ull;
+                if (more) next_row();
+            }
+            if (more) next = ld(min(b + l, e - 1u));
+            f(k, now, valid);
+            if (!more) break;
+        }
+    }
+};
+
 // ---------------------------------------------------------------------------------------
 // Wall collision.  Box: base_kernels.py:75-98.  Pipe: base_kernels.py:56-72, 101-127 and
 // util_kernels.py:38-204, in FP32, with the particle's own xoroshiro128+ stream.
@@ -810,6 +904,42 @@ __device__ __forceinline__ PairSums naive_pair_sums(const StepConsts& C, int i, 
     return S;
 }
 
+// The sums of the 64 / L particles that share a wavefront, over rows that they share: every lane
+// tests its candidate against each of them.
+template <int L>
+__device__ __forceinline__ PairSums shared_pair_sums(const SharedRows<64 / L>& rows, const StepConsts& C, int i,
+                                                     float4 p, float4 v, __amdgpu_buffer_rsrc_t rpos,
+                                                     __amdgpu_buffer_rsrc_t rvel) {
+    constexpr int P = 64 / L;
+    struct Pair { float4 q, v; };
+    PairSums S[P];
+    float4 ps[P], vs[P];  // the particles', the same in all lanes
+    uint32_t is[P];
+#pragma unroll
+    for (int j = 0; j < P; ++j) {
+        const int at = j * L;
+        ps[j] = make_float4(lane_of(p.x, at), lane_of(p.y, at), lane_of(p.z, at), lane_of(p.w, at));
+        vs[j] = make_float4(lane_of(v.x, at), lane_of(v.y, at), lane_of(v.z, at), 0.0f);
+        is[j] = (uint32_t)__builtin_amdgcn_readlane(i, at);
+    }
+    rows.walk([&](uint32_t k) { return Pair{ld_f4(rpos, k * 16u), ld_f4(rvel, k * 16u)}; },
+              [&](uint32_t k, const Pair& c, bool valid) {
+#pragma unroll
+                  for (int j = 0; j < P; ++j)
+                      if (valid && norm2(ps[j].x - c.q.x, ps[j].y - c.q.y, ps[j].z - c.q.z) <= C.h2 && k != is[j])
+                          S[j].add(C, ps[j], vs[j], c.q, c.v);
+              });
+    PairSums mine;
+    const int own = (int)(threadIdx.x & 63u) / L;
+#pragma unroll
+    for (int j = 0; j < P; ++j) {
+        const PairSums t{group_sum<64>(S[j].ax), group_sum<64>(S[j].ay), group_sum<64>(S[j].az),
+                         group_sum<64>(S[j].bx), group_sum<64>(S[j].by), group_sum<64>(S[j].bz)};
+        if (j == own) mine = t;
+    }
+    return mine;
+}
+
 // The same sums with L lanes per particle (L = 1 is naive_pair_sums): lane l of the group
 // walks list slots l, l + L, ... (and, past the list, every L-th candidate of each row), and
 // the partial sums are added across the group; every lane of the group returns the total.
@@ -827,6 +957,14 @@ __device__ __forceinline__ PairSums naive_pair_sums_lanes(const StepConsts& C, i
         const __amdgpu_buffer_rsrc_t rvel = make_rsrc(vel, (uint32_t)n * 16u);
         PairSums S;
         const uint32_t head = nn[i];
+        if constexpr (kSharesRows<L>) {
+            if (__ballot(head == kNoList) == ~0ull) {
+                const __amdgpu_buffer_rsrc_t rcs =
+                    make_rsrc(cs, ((uint32_t)C.cell_off + (uint32_t)C.n_cells + 1u) * 4u);
+                const SharedRows<64 / L> rows(p, C, rcs);
+                if (rows.ok) return shared_pair_sums<L>(rows, C, i, p, v, rpos, rvel);
+            }
+        }
         const uint32_t cnt = head < kNoList ? min(head, (uint32_t)kListCap) : 0u;
         // the lane's next list slot is loaded while this slot's neighbour is gathered
         uint32_t kn = l < cnt ? list_decode(nl[list_at(n, i, l)], i) : 0u;
