@@ -97,7 +97,7 @@ Layout plan_layout(const sph_ctx* c) {
     sz[S_PIDA] = sz[S_PIDB] = sz[S_RHOA] = 4 * nn;
     sz[S_KEYI] = sz[S_VALI] = sz[S_KEYS0] = sz[S_VALS0] = sz[S_KEYS1] = sz[S_VALS1] = 4 * nn;
     sz[S_CS] = 4 * ((size_t)c->sc.n_cells + 1);
-    sz[S_HIST] = 4 * 256 * (size_t)(c->num_tiles > 0 ? c->num_tiles : 1);
+    sz[S_HIST] = 4 * 256 * ((nn + 2047) / 2048);  // more and smaller tiles count in nn
     sz[S_DTOT] = 4 * 256;
     sz[S_RNG] = c->prm.mode == SPH_MODE_PIPE ? 16 * nn : 16;
     sz[S_DBGP] = sz[S_DBGV] = sz[S_DBGF] = c->keep_terms ? 16 * nn : 16;

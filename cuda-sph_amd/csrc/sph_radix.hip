@@ -236,21 +236,29 @@ __global__ __launch_bounds__(ST) void radix_downsweep(const uint32_t* __restrict
     }
 }
 
+// The tiles' digit counts.  tile_hist holds a tile per 2,048 keys; the counts of smaller tiles go to
+// the NAIVE formulation's list words, which the sort's contexts leave alone: 1 KiB per 512 keys
+// there, 4 B per particle.
+uint32_t* tile_counts(const sph_ctx* c) {
+    return (int64_t)c->num_tiles <= (c->n + 2047) / 2048 ? c->b.tile_hist : c->b.nn;
+}
+
 // One pass over the tiles.
 template <int SI, bool FEW>
 void launch_radix_pass(sph_ctx* c, int p, bool gather, const uint32_t* kin, const uint32_t* vin, uint32_t* kout,
                        uint32_t* vout, hipStream_t s) {
     const int n = (int)c->n, T = c->num_tiles, shift = c->pass_shift[p], bits = c->pass_bits[p];
     const Buffers& b = c->b;
-    radix_upsweep<SI, FEW><<<T, ST, 0, s>>>(kin, n, shift, (1u << bits) - 1u, b.tile_hist, T,
+    uint32_t* const counts = tile_counts(c);
+    radix_upsweep<SI, FEW><<<T, ST, 0, s>>>(kin, n, shift, (1u << bits) - 1u, counts, T,
                                            p == 0 ? b.flags + kFlagOutOfGrid : nullptr);
-    if (!FEW) radix_scan_digits<<<RADIX, ST, 0, s>>>(b.tile_hist, T, b.digit_total);
+    if (!FEW) radix_scan_digits<<<RADIX, ST, 0, s>>>(counts, T, b.digit_total);
     if (gather)
-        radix_downsweep<SI, FEW, true><<<T, ST, 0, s>>>(kin, vin, kout, vout, n, shift, bits, b.tile_hist,
+        radix_downsweep<SI, FEW, true><<<T, ST, 0, s>>>(kin, vin, kout, vout, n, shift, bits, counts,
                                                        b.digit_total, T, b.posB, b.velB, b.pidB, b.posA, b.velA,
                                                        b.pidA, c->sc, b.flags);
     else
-        radix_downsweep<SI, FEW, false><<<T, ST, 0, s>>>(kin, vin, kout, vout, n, shift, bits, b.tile_hist,
+        radix_downsweep<SI, FEW, false><<<T, ST, 0, s>>>(kin, vin, kout, vout, n, shift, bits, counts,
                                                         b.digit_total, T, nullptr, nullptr, nullptr, nullptr, nullptr,
                                                         nullptr, c->sc, nullptr);
 }
