@@ -403,9 +403,9 @@ struct RowWindows {
 // not wait for each batch in turn.  With 32 lanes, which rows rarely fill, the rows of one pass
 // over t are laid end to end and taken L at a time across their bounds; a lane finds its row from
 // the places where rows start, without LDS memory (20-step gradients of 16,384 particles
-// 1.575 -> 1.51 ms; with 16 lanes it lost 6% over the 64-box batch).  From the tail's start on,
-// without the candidates before the tail's first.  rows(k0, k1) gets the lane's own row ranges.
-template <int L, typename RowF, typename F>
+// 1.575 -> 1.51 ms; with 16 lanes it lost 6% over the 64-box batch).  Without AHEAD each row is
+// taken by itself and nothing is loaded before it is needed.  From the tail's start on, without the candidates before the tail's first.  rows(k0, k1) gets the lane's own row ranges.
+template <int L, bool AHEAD = true, typename RowF, typename F>
 __device__ __forceinline__ void for_each_batch(float px, float py, float pz, const StepConsts& C,
                                                __amdgpu_buffer_rsrc_t rcs, __amdgpu_buffer_rsrc_t rpos, uint32_t l,
                                                RowF&& rows, F&& f, ListTail tail = ListTail()) {
@@ -444,6 +444,16 @@ __device__ __forceinline__ void for_each_batch(float px, float py, float pz, con
                     q = ld_f4(rpos, k * 16u);
                 }
                 f(kc, qc, at + l < line.total);
+            }
+            continue;
+        }
+        if constexpr (!AHEAD) {
+            for (int j = 0; j < min(L, npairs - t0); ++j) {
+                const uint32_t k0 = __shfl(a0, gbase + j), k1 = __shfl(a1, gbase + j);
+                for (uint32_t b = k0; b < k1; b += L) {
+                    const uint32_t k = b + l;
+                    f(k, ld_f4(rpos, k * 16u), k < k1);
+                }
             }
             continue;
         }
@@ -532,8 +542,6 @@ struct SharedRows {
             RowGrid::range(C.cell_off + C.dims[0] * (cy + C.dims[1] * cz), q0, q1, C,
                            [&](int c) { return ld_u32(rcs, (uint32_t)c * 4u); }, k0, k1);
     }
-
-    __device__ __forceinline__ uint32_t candidates() const { return group_fold<64>(k0 < k1 ? k1 - k0 : 0u, [](uint32_t a, uint32_t b) { return a + b; }); }
 
     // f(k, ld(k), valid) by all 64 lanes together, lane l with the candidates k0 + l + 64 m of
     // each row; the next batch is loaded before f gets this one's

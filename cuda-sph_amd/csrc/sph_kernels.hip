@@ -196,18 +196,28 @@ struct StageBand {
     }
 };
 
+// Whether a particle's surroundings look dense enough for shared_density: its own row's candidates,
+// times its rows (at most about 1.7 times its candidates, a third of which are neighbours).  Costs
+// a pass over sparse particles 0.3 us (28,800 at 16 lanes); the shared rows outright cost 3.
+__device__ __forceinline__ bool crowded(const StepConsts& C, float4 p, __amdgpu_buffer_rsrc_t rcs) {
+    const RowGrid R(p.x, p.y, p.z, C);
+    const int cy = grid_coord(p.y, 1, C), cz = grid_coord(p.z, 2, C);
+    uint32_t q0, q1, k0 = 0u, k1 = 0u;
+    if (R.row(cy, R.rest_z(cz, C), C, q0, q1))
+        RowGrid::range(C.cell_off + C.dims[0] * (cy + C.dims[1] * cz), q0, q1, C,
+                       [&](int c) { return ld_u32(rcs, (uint32_t)c * 4u); }, k0, k1);
+    return (k1 - k0) * (uint32_t)((R.yhi - R.ylo + 1) * (R.zhi - R.zlo + 1)) >= 1024u;
+}
+
 // Density of the 64 / L particles that share a wavefront over rows that they share, if all of them
-// turn out to have more neighbours than a list and its tail serve (false: nothing is done).  Tried
-// from kSharedCandidates on, about a third of which are neighbours inside the fluid: 512 to 1,536
-// measured within 2% on the 64-box batch.
-constexpr uint32_t kSharedCandidates = 1024;
+// turn out to have more neighbours than a list and its tail serve (false: nothing is done).
 template <int L>
 __device__ __forceinline__ bool shared_density(const StepConsts& C, int i, uint32_t l, float4 p,
                                                __amdgpu_buffer_rsrc_t rpos, __amdgpu_buffer_rsrc_t rcs, float4* pos,
                                                float4* vel, float* __restrict__ rhoA, uint32_t* __restrict__ nn) {
     constexpr int P = 64 / L;
     const SharedRows<P> rows(p, C, rcs);
-    if (!rows.ok || rows.candidates() < kSharedCandidates) return false;
+    if (!rows.ok) return false;
     float x[P], y[P], z[P], acc[P];
     uint32_t cnt[P];
 #pragma unroll
@@ -262,8 +272,8 @@ constexpr uint32_t kOrderedTerms = 128;
 // (unique in the workgroup), gbase its group's first lane in the wavefront.  MASKED (L = 1): three
 // candidates at a time.  FAR (L = 1): lists beyond the int16 window too (kSeqList).  ORDERED (L > 1): the density is summed over the hits
 // in list order, as one lane sums it, to the same bits: the group keeps the hits' terms in terms
-// (kOrderedTerms words of LDS) and adds them up from there.
-template <int L, bool FAR = false, bool ORDERED = false, bool MASKED = false>
+// (kOrderedTerms words of LDS) and adds them up from there.  AHEAD (L > 1): see for_each_batch.
+template <int L, bool FAR = false, bool ORDERED = false, bool MASKED = false, bool AHEAD = true>
 __device__ __forceinline__ void density_particle(const StepConsts& G, const StepConsts& C, int i, uint32_t l,
                                                  StageBand<L> band, uint32_t gbase, float4* pos, float4* vel,
                                                  const uint32_t* __restrict__ cs, float* __restrict__ rhoA,
@@ -275,9 +285,7 @@ __device__ __forceinline__ void density_particle(const StepConsts& G, const Step
     const float4 p = pos[i];
     const size_t stride = (size_t)G.n;
     if constexpr (kSharesRows<L> && !ORDERED) {
-        if (__ballot(true) == ~0ull &&
-            shared_density<L>(C, i, l, p, rpos, make_rsrc(cs, ((uint32_t)G.cs_cells + 1u) * 4u), pos, vel, rhoA, nn))
-            return;
+        if (__ballot(crowded(C, p, rcs)) == ~0ull && shared_density<L>(C, i, l, p, rpos, rcs, pos, vel, rhoA, nn)) return;
     }
     float acc = 0.0f;
     uint32_t cnt = 0;
@@ -368,7 +376,7 @@ __device__ __forceinline__ void density_particle(const StepConsts& G, const Step
             kept = 0;
         };
         // one candidate per lane of the group, hits ranked by a ballot
-        for_each_batch<L>(
+        for_each_batch<L, AHEAD>(
             p.x, p.y, p.z, C, rcs, rpos, l,
             [&](uint32_t k0, uint32_t k1) {
                 klo = min(klo, k0);
@@ -420,7 +428,7 @@ __device__ __forceinline__ void density_particle(const StepConsts& G, const Step
 
 // Plain step: L lanes per particle (1, 2, 4, 8, 16, 32 or 64), particle gt / L.  Groups are aligned,
 // so a whole group leaves together at the end of the range.
-template <int L, bool FAR = false, bool ORDERED = false, bool MASKED = false>
+template <int L, bool FAR = false, bool ORDERED = false, bool MASKED = false, bool AHEAD = true>
 __global__ __launch_bounds__(kDensityThreads) void naive_density_kernel(StepConsts G, float4* pos, float4* vel,
                                                                          const uint32_t* __restrict__ cs,
                                                                          float* __restrict__ rhoA,
@@ -434,7 +442,7 @@ __global__ __launch_bounds__(kDensityThreads) void naive_density_kernel(StepCons
     const uint32_t lane = threadIdx.x & 63u;
     const StageBand<L> band{s_stage[threadIdx.x >> 6], lane / L};
     __shared__ __align__(16) float s_terms[ORDERED ? kDensityThreads / L : 1][ORDERED ? kOrderedTerms : 1];
-    density_particle<L, FAR, ORDERED, MASKED>(G, G, i, gt & (L - 1), band, lane & ~(uint32_t)(L - 1), pos, vel, cs, rhoA, nl, nn,
+    density_particle<L, FAR, ORDERED, MASKED, AHEAD>(G, G, i, gt & (L - 1), band, lane & ~(uint32_t)(L - 1), pos, vel, cs, rhoA, nl, nn,
                                       s_terms[ORDERED ? threadIdx.x / L : 0]);
 }
 
@@ -1086,11 +1094,18 @@ hipError_t launch_rekey(sph_ctx* c, hipStream_t s) {
     return hipGetLastError();
 }
 
-template <int L, bool FAR = false, bool ORDERED = false, bool MASKED = false>
+// Up to this many threads groups of 2 and 4 lanes load a batch of candidates ahead (for_each_batch);
+// they take many batches per row, and with more wavefronts to hide the loads the bookkeeping
+// costs more.  us per launch, ahead / not: box of 65,537 particles at 4 lanes 24.6 / 25.8, 80,000
+// at 2 40.3 / 42.2, dam break of 42,000 at 4 19.8 / 23.8; of 137,500 at 2 42.0 / 38.1, 112,500 at 4
+// 32.4 / 28.0, 211,420 at 2 51.5 / 44.0.  Batches always look ahead (the 64 boxes 508 / 527).
+constexpr int64_t kAheadThreads = 270000;
+
+template <int L, bool FAR = false, bool ORDERED = false, bool MASKED = false, bool AHEAD = true>
 void launch_density_lanes(sph_ctx* c, hipStream_t s) {
     const int bs = c->density_block;
     const Buffers& b = c->b;
-    naive_density_kernel<L, FAR, ORDERED, MASKED><<<blocks_for(c->n * L, bs), bs, 0, s>>>(c->sc, b.posA, b.velA, b.cs, b.rhoA, b.nl, b.nn);
+    naive_density_kernel<L, FAR, ORDERED, MASKED, AHEAD><<<blocks_for(c->n * L, bs), bs, 0, s>>>(c->sc, b.posA, b.velA, b.cs, b.rhoA, b.nl, b.nn);
 }
 
 // Most lanes of an instance: up to 16, the batch's passes leave out what 32 and 64 lanes need
@@ -1123,8 +1138,14 @@ hipError_t launch_density(sph_ctx* c, hipStream_t s) {
         return hipGetLastError();
     }
     switch (c->lanes) {
-        case 2: launch_density_lanes<2>(c, s); break;
-        case 4: launch_density_lanes<4>(c, s); break;
+        case 2:
+            if (c->n * 2 <= kAheadThreads) launch_density_lanes<2>(c, s);
+            else launch_density_lanes<2, false, false, false, false>(c, s);
+            break;
+        case 4:
+            if (c->n * 4 <= kAheadThreads) launch_density_lanes<4>(c, s);
+            else launch_density_lanes<4, false, false, false, false>(c, s);
+            break;
         case 8: launch_density_lanes<8>(c, s); break;
         case 16: launch_density_lanes<16>(c, s); break;
         case 32: launch_density_lanes<32>(c, s); break;

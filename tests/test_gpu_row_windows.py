@@ -34,3 +34,18 @@ def test_windows_over_rows_find_every_neighbour(gpu, lanes, n, mean, scale):
     got, want = batch.download()[0], plain(lanes, 3)
     for f in ("position", "velocity", "density"):
         assert np.array_equal(getattr(got, f), getattr(want, f)), f
+
+
+# groups of 2 and 4 lanes look a batch ahead up to 270,000 threads and in batches: the same bits
+@pytest.mark.parametrize("lanes,n", [(2, 135000), (2, 135001), (4, 67500), (4, 67501)])
+def test_plain_groups_and_batches_sum_alike(gpu, lanes, n):
+    h = (30 / (n / 0.4 ** 3) / (4.0 / 3.0 * np.pi)) ** (1.0 / 3.0)
+    w = box_uniform(n, seed=87, h=h)
+    state = SimulationState(w.state.position, np.random.default_rng(88).normal(0.0, 0.3, size=(n, 3)), np.zeros(n))
+    batch = BatchedSPH([(w.params, w.constants)], device=gpu, lanes=[lanes])
+    batch.upload([state])
+    batch.step(2)
+    got = batch.download()[0]
+    want = NaiveSPHStrategy(w.params, constants=w.constants, device=gpu, lanes=lanes).advance(state, 2)
+    for f in ("position", "velocity", "density"):
+        assert np.array_equal(getattr(got, f), getattr(want, f)), f
