@@ -478,7 +478,7 @@ __device__ __forceinline__ BatchLane batch_lane(const StepConsts& G, uint32_t gt
 
 // TOP, 16 or 64, is the largest group that the kernel has code for: the path of 32 lanes over rows
 // laid end to end costs the others 4% where it stands beside them (64 boxes of 2,048 to 65,536
-// particles at up to 16 lanes, 4 steps: 5.98 ms, 5.74 without it).  A larger group than TOP, which
+// particles at up to 16 lanes, 4 steps, before these shared rows: 5.98 ms, 5.74 without it).  A larger group than TOP, which
 // a graph captured before the lanes were set can meet, works with its first TOP lanes.
 template <int TOP>
 __global__ __launch_bounds__(kDensityThreads) void naive_density_batch_kernel(StepConsts G, float4* pos, float4* vel,
@@ -515,8 +515,8 @@ __global__ __launch_bounds__(kDensityThreads) void naive_density_batch_kernel(St
 
 // Force pass (naive_kernels.py:24-80) fused with integration and collision: each lane
 // walks its particle's neighbour list (one coalesced load per slot, kForceUnroll slots and
-// their gathers in flight); a particle with more neighbours than list slots rescans its
-// candidates instead.  With L lanes per particle the group splits the list (or the rescan)
+// their gathers in flight); a particle with more neighbours than list slots scans its list's
+// tail or all of its candidates instead.  With L lanes per particle the group splits the list (or the rescan)
 // and lane 0 finishes the particle.  MODE selects the wall collision at compile time.
 template <int MODE, int L = 1, bool COUNT = false, bool ORDERED = false>
 __global__ __launch_bounds__(256) void naive_force_kernel(
@@ -1051,11 +1051,19 @@ int ordered_lanes(const sph_ctx* c) {
     return c->n <= 24576 ? 16 : c->n <= 98304 ? 8 : 1;
 }
 
-// Up to this many particles the VOXEL density pass gives each 32 lanes; past that the card is full
-// with one.  us per launch, one lane / 32: box of 4,096 particles 41.5 / 8.6, 16,384 36.8 / 11.4,
-// 40,000 47.2 / 20.9, 65,536 54.9 / 32.6, 98,304 65.1 / 48.0, 131,072 42.7 / 45.4, 262,144
-// 59.4 / 88.5; dam break of 55,296 47.5 / 29.4, 119,621 37.5 / 44.4.
-constexpr int64_t kVoxelGroupParticles = 98304;
+// Whether the VOXEL density pass gives each particle 32 lanes: up to a particle count from which the
+// card is full with one, which lies higher the more candidates the voxels hold, that is the
+// longer their edges are against h.  us per launch, one lane / 32, at h of
+//     1 to 1.9 edges    box of 65,536 54.9 / 32.6, 98,304 65.1 / 48.0, 131,072 42.7 / 45.4, 262,144
+//                       59.4 / 88.5; dam break of 55,296 47.5 / 29.4, 96,256 36.0 / 33.8
+//     0.5 to 0.95       dam break of 66,048 169 / 48, 96,256 66 / 46, 131,072 75 / 68, 307,200
+//                       174.0 / 173.4
+//     less              24,576 375 / 35, 131,072 298 / 128, 307,200 733 / 411
+bool voxel_groups(const sph_ctx* c) {
+    const float edge = fmaxf(c->sc.cell[0], fmaxf(c->sc.cell[1], c->sc.cell[2]));
+    const float h = c->sc.h;
+    return c->n <= (h >= 0.95f * edge ? 98304 : h >= 0.5f * edge ? 131072 : 307200);
+}
 
 hipError_t launch_fill_u32(uint32_t* p, uint32_t v, int64_t n, hipStream_t s) {
     if (n > 0) fill_u32_kernel<<<blocks_for(n, 256), 256, 0, s>>>(p, v, n);
@@ -1119,7 +1127,7 @@ int batch_top_lanes(const sph_ctx* c) {
 hipError_t launch_density(sph_ctx* c, hipStream_t s) {
     if (c->n == 0) return hipGetLastError();
     const int bs = c->density_block;
-    if (c->sc.formulation == SPH_FORM_VOXEL && c->n <= kVoxelGroupParticles) {
+    if (c->sc.formulation == SPH_FORM_VOXEL && voxel_groups(c)) {
         voxel_density_group_kernel<<<blocks_for(c->n * kVoxelGroup, bs), bs, 0, s>>>(
             c->sc, c->b.posA, c->b.velA, c->b.cs, c->b.rhoA, c->b.nbr, c->b.flags);
         return hipGetLastError();

@@ -1,4 +1,6 @@
 """VOXEL density by 32 lanes per particle, which few particles take, against the one-lane kernel."""
+from dataclasses import replace
+
 import numpy as np
 import pytest
 
@@ -37,5 +39,25 @@ def test_voxel_groups_equal_one_lane(gpu, n, mean, form, block):
         return sim.advance(SimulationState(pos[:count], vel[:count], np.zeros(count)), 1)
 
     want, got = run(ONE_LANE), run(n)
+    for f in ("position", "velocity", "density"):
+        assert np.array_equal(getattr(got, f), getattr(want, f)[:n], equal_nan=True), f
+
+
+# with h from 0.5 to 0.95 of the voxel's edge up to 131,072 particles have groups, below that 307,200
+@pytest.mark.parametrize("n,edges,most", [(131072, 0.7, 131072), (20011, 0.7, 131072), (307200, 0.4, 307200),
+                                          (20011, 0.2, 307200)])
+def test_coarse_voxels_equal_one_lane(gpu, n, edges, most):
+    h = (30 / (n / 0.4 ** 3) / (4.0 / 3.0 * np.pi)) ** (1.0 / 3.0)
+    w = box_uniform(most + 1, seed=89, h=h)
+    rng = np.random.default_rng(90)
+    pos, vel = w.state.position, rng.normal(0.0, 0.3, size=(most + 1, 3))
+    pos[n:] = rng.uniform(0.7, 0.95, size=(most + 1 - n, 3))
+
+    def run(count):
+        params = replace(box_uniform(count, h=h).params, voxel_size=np.array([h / edges] * 3))
+        sim = VoxelSPHStrategy(params, constants=w.constants, device=gpu, check_finite=False)
+        return sim.advance(SimulationState(pos[:count], vel[:count], np.zeros(count)), 1)
+
+    want, got = run(most + 1), run(n)
     for f in ("position", "velocity", "density"):
         assert np.array_equal(getattr(got, f), getattr(want, f)[:n], equal_nan=True), f
