@@ -800,6 +800,17 @@ __global__ __launch_bounds__(256) void voxel_density_group_kernel(StepConsts C, 
     if (first + mine < C.n && slot < s_count[mine]) nbr[(size_t)(1 + slot) * (size_t)C.n + first + mine] = s_list[mine][slot];
 }
 
+// Coefficients of one pair's pressure term (of x_i - x_j) and viscosity term (of v_j - v_i).
+__device__ __forceinline__ void voxel_pair(const StepConsts& C, float fi, float s, float r2, float pj, float ij,
+                                           float& cp, float& cv) {
+    const float r = sqrtf(r2);
+    const float hr = C.h - r;
+    // voxel_kernels.py:162-168: (p_i/rho_i^2 + p_j/rho_j^2) * grad W
+    cp = (fi + pj * ij * ij) * C.grad_c * hr * hr * (1.0f / r);
+    // voxel_kernels.py:203-208: (v_j - v_i) / rho_j * lap W * m * mu / rho_i
+    cv = ij * (C.lap_c * hr) * s;
+}
+
 template <int MODE>
 __global__ __launch_bounds__(256) void voxel_force_kernel(
     StepConsts C, const float4* __restrict__ pos, const float4* __restrict__ vel, const uint32_t* __restrict__ pidA,
@@ -833,15 +844,11 @@ __global__ __launch_bounds__(256) void voxel_force_kernel(
             if (t0 + u >= cnt || jj[u] == i) continue;
             const float4 q = qq[u], vj = vv[u];
             const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
-            const float r = sqrtf(norm2(dx, dy, dz));
-            const float hr = C.h - r;
-            // voxel_kernels.py:162-168: (p_i/rho_i^2 + p_j/rho_j^2) * grad W
-            const float cp = (fi + q.w * vj.w * vj.w) * C.grad_c * hr * hr * (1.0f / r);
+            float cp, cv;
+            voxel_pair(C, fi, s, norm2(dx, dy, dz), q.w, vj.w, cp, cv);
             ax += cp * dx;
             ay += cp * dy;
             az += cp * dz;
-            // voxel_kernels.py:203-208: (v_j - v_i) / rho_j * lap W * m * mu / rho_i
-            const float cv = vj.w * (C.lap_c * hr) * s;
             bx += (vj.x - v.x) * cv;
             by += (vj.y - v.y) * cv;
             bz += (vj.z - v.z) * cv;
@@ -850,6 +857,60 @@ __global__ __launch_bounds__(256) void voxel_force_kernel(
     // voxel_kernels.py:211 min(1, .)
     const Vec3 V{fminf(1.0f, bx), fminf(1.0f, by), fminf(1.0f, bz)};
     finish_particle<MODE, false>(C, i, p, v, pidA[i], rho_i, Vec3{ax, ay, az}, V, posOut, velOut, pidOut, keyI, valI, rng, pipe,
+                    dbgP, dbgV, dbgF, flags);
+}
+
+// The same sums and bits by 32 lanes per particle, for few particles: a lane per list entry works out
+// its pair's terms, and six lanes add one component each in list order (as
+// naive_pair_sums_ordered does), so that a list is one wait, not eight (kVoxelForceGroups).
+template <int MODE>
+__global__ __launch_bounds__(256) void voxel_force_group_kernel(
+    StepConsts C, const float4* __restrict__ pos, const float4* __restrict__ vel, const uint32_t* __restrict__ pidA,
+    const float* __restrict__ rhoA, const int32_t* __restrict__ nbr, float4* __restrict__ posOut,
+    float4* __restrict__ velOut, uint32_t* __restrict__ pidOut, uint32_t* __restrict__ keyI,
+    uint32_t* __restrict__ valI, uint64_t* __restrict__ rng,
+    const PipeTable* __restrict__ pipe, float4* __restrict__ dbgP, float4* __restrict__ dbgV,
+    float4* __restrict__ dbgF, uint32_t* __restrict__ flags) {
+    constexpr uint32_t kPitch = kOrderedPitch<kVoxelGroup>;
+    __shared__ float s_pairs[256 / kVoxelGroup][kOrderedPairWords<kVoxelGroup>];
+    const int i = (int)((xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x) / kVoxelGroup);
+    if (i >= C.n) return;  // the whole group
+    const uint32_t l = threadIdx.x & 31u;
+    const int gbase = (int)(threadIdx.x & 32u);
+    const size_t n = (size_t)C.n;
+    const float4 p = pos[i], v = vel[i];
+    const int cnt = nbr[i];
+    const float rho_i = rhoA[i];
+    const float fi = p.w / (rho_i * rho_i);
+    const float s = C.mass * C.visc / rho_i;
+    float* const buf = s_pairs[threadIdx.x / kVoxelGroup];
+    if ((int)l < cnt) {
+        const int j = nbr[(size_t)(1 + l) * n + i];
+        const float4 q = pos[j], vj = vel[j];
+        const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
+        float cp, cv;
+        voxel_pair(C, fi, s, norm2(dx, dy, dz), q.w, vj.w, cp, cv);
+        const bool self = j == i;  // left out: nothing times nothing
+        buf[l] = self ? 0.0f : cp;
+        buf[kPitch + l] = self ? 0.0f : cv;
+        buf[2u * kPitch + l] = self ? 0.0f : dx;
+        buf[3u * kPitch + l] = self ? 0.0f : dy;
+        buf[4u * kPitch + l] = self ? 0.0f : dz;
+        buf[5u * kPitch + l] = self ? 0.0f : vj.x - v.x;
+        buf[6u * kPitch + l] = self ? 0.0f : vj.y - v.y;
+        buf[7u * kPitch + l] = self ? 0.0f : vj.z - v.z;
+    }
+    __builtin_amdgcn_wave_barrier();
+    const uint32_t comp = l < 6u ? l : 5u;
+    const float* const coef = buf + (comp < 3u ? 0u : kPitch);
+    const float* const part = buf + (2u + comp) * kPitch;
+    float acc = 0.0f;
+    for (int t = 0; t < cnt; ++t) acc += coef[t] * part[t];
+    const Vec3 P{__shfl(acc, gbase), __shfl(acc, gbase + 1), __shfl(acc, gbase + 2)};
+    const float bx = __shfl(acc, gbase + 3), by = __shfl(acc, gbase + 4), bz = __shfl(acc, gbase + 5);
+    if (l != 0u) return;
+    const Vec3 V{fminf(1.0f, bx), fminf(1.0f, by), fminf(1.0f, bz)};  // voxel_kernels.py:211
+    finish_particle<MODE, false>(C, i, p, v, pidA[i], rho_i, P, V, posOut, velOut, pidOut, keyI, valI, rng, pipe,
                     dbgP, dbgV, dbgF, flags);
 }
 
@@ -1065,6 +1126,11 @@ bool voxel_groups(const sph_ctx* c) {
     return c->n <= (h >= 0.95f * edge ? 98304 : h >= 0.5f * edge ? 131072 : 307200);
 }
 
+// Up to this many particles the VOXEL force pass gives each 32 lanes.  us per launch, one lane / 32
+// (dam break): 4,096 particles 12.6 / 6.3, 16,512 14.1 / 9.9, 24,576 13.4 / 11.9, 32,768 14.2 / 13.8,
+// 55,296 14.1 / 18.3.
+constexpr int64_t kVoxelForceGroups = 32768;
+
 hipError_t launch_fill_u32(uint32_t* p, uint32_t v, int64_t n, hipStream_t s) {
     if (n > 0) fill_u32_kernel<<<blocks_for(n, 256), 256, 0, s>>>(p, v, n);
     return hipGetLastError();
@@ -1190,7 +1256,9 @@ void launch_force_mode(sph_ctx* c, hipStream_t s, bool count) {
     float4* dV = c->keep_terms ? c->b.dbgV : nullptr;
     float4* dF = c->keep_terms ? c->b.dbgF : nullptr;
     if (c->sc.formulation == SPH_FORM_VOXEL) {
-        voxel_force_kernel<MODE><<<blocks_for(c->n, bs), bs, 0, s>>>(
+        const bool groups = c->n <= kVoxelForceGroups;
+        const auto kernel = groups ? voxel_force_group_kernel<MODE> : voxel_force_kernel<MODE>;
+        kernel<<<blocks_for(groups ? c->n * kVoxelGroup : c->n, bs), bs, 0, s>>>(
             c->sc, c->b.posA, c->b.velA, c->b.pidA, c->b.rhoA, c->b.nbr, c->b.posB, c->b.velB, c->b.pidB, c->b.keyI,
             c->b.valI, c->b.rng, c->b.pipe, dP, dV, dF, c->b.flags);
         return;

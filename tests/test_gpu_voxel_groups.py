@@ -1,4 +1,5 @@
-"""VOXEL density by 32 lanes per particle, which few particles take, against the one-lane kernel."""
+"""VOXEL density and force by 32 lanes per particle, which few particles take, against the one-lane
+kernels."""
 from dataclasses import replace
 
 import numpy as np
@@ -10,13 +11,14 @@ from sph_amd.workloads import box_uniform
 
 pytestmark = pytest.mark.gpu
 
-ONE_LANE = 98305  # the fewest particles of the one-lane kernel
+ONE_LANE = 98305  # the fewest particles of the one-lane density kernel; the force kernel's are 32,769
 
 
 # 2 and 60 neighbours end before and after the 32 a list holds; "pile" puts all particles into one
 # voxel, "outside" some out of the grid, whose keys wrap (no voxel may be skipped then)
 @pytest.mark.parametrize("n,mean,form", [(1, 30, ""), (7, 2, ""), (9, 60, ""), (3001, 2, ""), (3001, 30, ""), (3001, 60, ""),
-                                         (700, 30, "pile"), (3001, 30, "outside"), (98303, 30, "")])
+                                         (700, 30, "pile"), (3001, 30, "outside"), (32768, 60, ""), (32769, 30, ""),
+                                         (98303, 30, "")])
 @pytest.mark.parametrize("block", [64, 256])
 def test_voxel_groups_equal_one_lane(gpu, n, mean, form, block):
     """Particles too far away to be anyone's neighbour bring the state past the group kernel's range;
