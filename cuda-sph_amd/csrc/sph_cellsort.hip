@@ -323,67 +323,167 @@ __global__ __launch_bounds__(CT) void cell_order_kernel(int n, SlabTable T, cons
 // collects those in it, scans its cells' counts, places its particles cell by cell in LDS,
 // orders each cell there and gathers its part of the state, and writes its part of the table.
 // The passes above take five launches of about 4.4 us each at these sizes, whatever their work,
-// and atomics in the force pass; this one takes 6 us with 4,096 particles (two launches before,
-// 12.4), 8 with 16,384 (23), 12 with 65,537 (18).  What bounds it is one latency after another
-// (keys, ids, state), and for many particles the keys' 4 n bytes in each of 256 workgroups.
-// A range with more than kOneList particles is collected in global memory (tmpE, tmpK) instead,
-// by a second walk over the keys.  A cell of more than kHeavyCell particles is ordered through a
-// bitmap of its (slab, id) in place of comparing each with each, which one workgroup alone
-// would take long for (70,000 particles in one cell: 5e9 comparisons).
+// and atomics in the force pass.  What bounds this one is one latency after another (keys, ids,
+// state), and for many particles the keys' 4 n bytes in each workgroup.
+// Where the particles crowd (a pile, a layer at one end of z), a range is cut into parts, which
+// further workgroups take: each works the cut out for itself, from one key per thread, spread
+// over all of them.  us per sort with the passes above / one workgroup per range / with the
+// cut: 65,537 particles in the first cells of 1,048,576, 30 in each, 24 / 622 / 23, 500 in each
+// 85 / 3,264 / 64; a layer of 5% of z, 19 / 40 / 19.  Particles that do not crowd pay 0.3 us
+// (5,000) to 1 us (65,537) for the look at the sample.
+// A range or part with more than `list` particles is collected in global memory (tmpE, tmpK)
+// instead, by a second walk over the keys.  A cell of more than kHeavyCell particles is ordered
+// through a bitmap of its (slab, id) in place of comparing each with each, which one workgroup
+// alone would take long for (70,000 particles in one cell: 5e9 comparisons).
 constexpr int OT = 1024;
 constexpr int OWAVES = OT / 64;
-constexpr int kOneGroups = 256;  // one per CU
-constexpr int kOneList = 2048;   // particles of a workgroup's range kept in LDS
-constexpr int kOneCells = 4096;  // cells of a range, at most
+constexpr int kOneGroups = 256;  // workgroups: one per CU
+constexpr int kOneMost = 1 << 20;  // cells, at most
+constexpr int kOneShares = 48;   // shares of all particles that ranges are measured by, at most ...
+constexpr int kOneShare = 1024;  // ... and particles of one, at least
+constexpr int kOneList = 3072;   // particles of a range or part kept in LDS ...
+constexpr int kOneAll = 4096;    // ... all of them up to this many
 constexpr int kOneLoads = 4;     // 16-byte key loads in flight per lane
 constexpr int kHeavyCell = 512;
-// step with the passes above against this one (30 neighbours, 4 lanes): 30.6 against 25.4 us with
-// 16,384 particles, 40.6 / 38.6 with 49,152, 45.3 / 44.6 with 65,537, 51.3 / 51.9 with 81,920
+// us per step with the passes above / this one (30 neighbours, 4 lanes), in a corner of the box and all
+// over it: 16,384 particles 39.9 / 32.3 and 40.0 / 32.2, 49,152 44.8 / 40.6 and 43.9 / 37.9, 65,537
+// 48.8 / 47.1 and 46.1 / 42.0, 73,728 52.6 / 53.4 and 46.3 / 44.1
 constexpr int64_t kOneSort = 73728;
 constexpr int kHeavyMost = (int)(kOneSort / (kHeavyCell + 1)) + 1;  // heavy cells of a range, at most
 inline __host__ __device__ int heavy_words(int n, bool slabs) { return ((slabs ? 4 : 1) * n + 31) / 32; }
+inline __host__ __device__ int one_list(int n) { return n <= kOneAll ? kOneAll : kOneList; }
+inline __host__ __device__ int one_shares(int n) { return n <= kOneAll ? 0 : min(kOneShares, n / kOneShare); }
+// Parts of a range that holds `seen` of the OT sampled keys: one up to two shares of them, past that
+// a part per share (rounded up), so that over all ranges the parts past the first are at most
+// `shares`.
+__device__ __forceinline__ uint32_t one_parts(uint32_t seen, int shares) {
+    const uint32_t x = seen * (uint32_t)shares;
+    return x > 2u * OT ? (x + OT - 1u) / OT : 1u;
+}
+
+// The range and the part of it that is the h-th of the parts past the first, from the sampled keys
+// per range; range -1: there are fewer.  One wavefront, lane l the ranges 4 l .. 4 l + 3.
+__device__ __forceinline__ void one_share(const uint32_t* hist, int ranges, int shares, int h, int* out) {
+    static_assert(kOneGroups == 256, "four ranges per lane");
+    const int lane = threadIdx.x & 63;
+    uint32_t more[4], sum = 0u;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        more[u] = 4 * lane + u < ranges ? one_parts(hist[4 * lane + u], shares) - 1u : 0u;
+        sum += more[u];
+    }
+    uint32_t first = wave_incl_scan(sum) - sum;
+    if (lane == 63 && (uint32_t)h >= first + sum) out[0] = -1;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        if ((uint32_t)h >= first && (uint32_t)h < first + more[u]) {
+            out[0] = 4 * lane + u;
+            out[1] = h - (int)first + 1;
+        }
+        first += more[u];
+    }
+}
 
 template <bool GATHER>
 __global__ __launch_bounds__(OT) void cell_sort_one_kernel(
-    int n, int m, int per, SlabTable T, const uint32_t* __restrict__ keyI, const uint32_t* __restrict__ pidB,
-    uint32_t* __restrict__ cs, uint32_t* __restrict__ skey, uint32_t* __restrict__ sval,
-    const float4* __restrict__ posB, const float4* __restrict__ velB, float4* __restrict__ posA,
-    float4* __restrict__ velA, uint32_t* __restrict__ pidA, uint32_t* tmpE, uint32_t* tmpK) {
+    int n, int m, int per, int ranges, SlabTable T, const uint32_t* __restrict__ keyI,
+    const uint32_t* __restrict__ pidB, uint32_t* __restrict__ cs, uint32_t* __restrict__ skey,
+    uint32_t* __restrict__ sval, const float4* __restrict__ posB, const float4* __restrict__ velB,
+    float4* __restrict__ posA, float4* __restrict__ velA, uint32_t* __restrict__ pidA, uint32_t* tmpE, uint32_t* tmpK) {
     extern __shared__ uint32_t s_one[];
-    uint32_t* const start = s_one;             // per + 1: a cell's first place in the range
-    uint32_t* const cur = start + per + 1;     // per: its count, then its next free place
-    uint32_t* const table = cur + per;         // per: its table entry
-    uint32_t* const listE = table + per;       // kOneList: the range's particles (slots) as found ...
-    uint32_t* const listK = listE + kOneList;  // ... their keys
-    uint32_t* const ordE = listK + kOneList;   // ... cell by cell
-    uint32_t* const ordK = ordE + kOneList;    // ... (slab, id) there
-    uint32_t* const bits = ordK + kOneList;    // heavy_words: a heavy cell's (slab, id)
+    const int list = one_list(n), shares = one_shares(n);
+    uint32_t* const start = s_one;          // per + 1: a cell's first place in the range
+    uint32_t* const cur = start + per + 1;  // per: its count, its next free place, its table entry's fields
+    uint32_t* const ordE = cur + per;       // list: the range's particles (slots) cell by cell
+    uint32_t* const ordK = ordE + list;     // ... (slab, id) there
+    uint32_t* const listE = ordK + list;    // ... as found
+    uint32_t* const listK = listE + list;   // ... their keys
+    uint32_t* const bits = listE;           // heavy_words, after that: a heavy cell's (slab, id)
     __shared__ uint32_t s_wave[OWAVES], s_count, s_below, s_heavy, s_cell[kHeavyMost], s_ones[OT];
+    __shared__ uint32_t s_hist[kOneGroups], s_seen;
+    __shared__ int s_share[2], s_lo, s_hi;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int lo = xcd_tile(blockIdx.x, gridDim.x) * per, hi = min(lo + per, m);  // this range of cells
-    if (lo >= hi) return;
-    const int own = hi - lo;
-    for (int c = tid; c < own; c += OT) cur[c] = 0u;
-    if (tid == 0) s_count = s_below = s_heavy = 0u;
-    __syncthreads();
-    uint32_t below = 0u;
     auto cell_of = [&](uint32_t key) { return (int)(key & kCellKeyMask); };
+    // this thread's sample of the keys: four neighbours share one of 256 places
+    const int sample = shares > 0 ? cell_of(keyI[(tid / 4) * (n / 4) / (OT / 4) * 4 + tid % 4]) : 0;
+    const uint4* const key4 = reinterpret_cast<const uint4*>(keyI);
+    const int quads = n / 4;
+    uint4 k[kOneLoads] = {};
+    auto load = [&](int v0) {
+#pragma unroll
+        for (int u = 0; u < kOneLoads; ++u) k[u] = key4[min(v0 + u * OT, quads - 1)];
+    };
+    if (quads > 0) load(tid);  // while the samples are looked at
+    for (int c = tid; c < per; c += OT) cur[c] = 0u;
+    if (tid == 0) s_count = s_below = s_heavy = s_seen = 0u;
+    const int block = xcd_tile(blockIdx.x, gridDim.x);
+    int range = block, part = 0;
+    if (block >= ranges) {
+        for (int r = tid; r < kOneGroups; r += OT) s_hist[r] = 0u;
+        __syncthreads();
+        atomicAdd(&s_hist[sample / per], 1u);
+        __syncthreads();
+        if (w == 0) one_share(s_hist, ranges, shares, block - ranges, s_share);
+        __syncthreads();
+        range = s_share[0];
+        part = s_share[1];
+        if (range < 0) return;
+    }
+    int lo = range * per, hi = min(lo + per, m);  // this range of cells
     auto mine = [&](int c) { return c >= lo && c < hi; };
+    __syncthreads();
+    if (shares > 0) {
+        const uint32_t found = (uint32_t)__popcll(__ballot(mine(sample)));
+        if (lane == 0 && found) atomicAdd(&s_seen, found);
+        __syncthreads();
+        const uint32_t seen = s_seen, parts = one_parts(seen, shares);
+        if (parts > 1u) {  // the part's: the cells before which its share of the range's samples lies
+            const int cells = hi - lo;
+            if (mine(sample)) atomicAdd(&cur[sample - lo], 1u);
+            if (tid == 0) s_lo = s_hi = cells;
+            __syncthreads();
+            const int each = (cells + OT - 1) / OT;
+            const int c0 = min(tid * each, cells), c1 = min(c0 + each, cells);
+            uint32_t sum = 0u;
+            for (int c = c0; c < c1; ++c) sum += cur[c];
+            const uint32_t incl = wave_incl_scan(sum);
+            if (lane == 63) s_wave[w] = incl;
+            __syncthreads();
+            uint32_t run = incl - sum;
+            for (int j = 0; j < w; ++j) run += s_wave[j];
+            const float rate = (float)parts / (float)seen;
+            auto part_of = [&](uint32_t before) { return min((int)((float)before * rate), (int)parts - 1); };
+            // the wavefront's first cell of this part or a later one, and of a later one
+            auto bound = [&](int least, int* at) {
+                const uint64_t found = __ballot(c0 < c1 && part_of(run + sum) >= least);
+                if (!found || lane != __ffsll((unsigned long long)found) - 1) return;
+                uint32_t before = run;
+                int c = c0;
+                while (c < c1 && part_of(before) < least) before += cur[c++];
+                atomicMin(at, c);
+            };
+            if (part > 0) bound(part, &s_lo);
+            bound(part + 1, &s_hi);
+            __syncthreads();
+            hi = lo + s_hi;
+            lo += part > 0 ? s_lo : 0;
+            for (int c = tid; c < cells; c += OT) cur[c] = 0u;
+            __syncthreads();
+        }
+    }
+    const int own = hi - lo;
+    uint32_t below = 0u;
     auto take = [&](uint32_t key, int c, int e) {
         atomicAdd(&cur[c - lo], 1u);
         const uint32_t at = atomicAdd(&s_count, 1u);
-        if (at < (uint32_t)kOneList) {
+        if (at < (uint32_t)list) {
             listE[at] = (uint32_t)e;
             listK[at] = key;
         }
     };
     // most quads hold no key of the range
-    const uint4* const key4 = reinterpret_cast<const uint4*>(keyI);
-    const int quads = n / 4;
     for (int v0 = tid; v0 < quads; v0 += kOneLoads * OT) {
-        uint4 k[kOneLoads];
-#pragma unroll
-        for (int u = 0; u < kOneLoads; ++u) k[u] = key4[min(v0 + u * OT, quads - 1)];
+        if (v0 != tid) load(v0);
 #pragma unroll
         for (int u = 0; u < kOneLoads; ++u) {
             const int v = v0 + u * OT;
@@ -419,11 +519,9 @@ __global__ __launch_bounds__(OT) void cell_sort_one_kernel(
     __syncthreads();
     uint32_t run = incl - sum;
     for (int k = 0; k < w; ++k) run += s_wave[k];
-    const uint32_t empty = T.empty();
     for (int c = c0; c < c1; ++c) {
         const uint32_t v = cur[c];
         start[c] = run;
-        table[c] = (base + run) | (v == 0u ? empty : 0u);
         cur[c] = run;
         run += v;
         if (v > (uint32_t)kHeavyCell) s_cell[atomicAdd(&s_heavy, 1u)] = (uint32_t)c;
@@ -453,7 +551,7 @@ __global__ __launch_bounds__(OT) void cell_sort_one_kernel(
         // particle E[at] of cell c: r of its particles come before it, b_j are in slabs below j
         auto put = [&](uint32_t at, int c, uint32_t r, uint32_t b1, uint32_t b2, uint32_t b3) {
             const uint32_t e = E[at], f = base + start[c] + r;
-            if (slabs && r == 0u) table[c] |= slab_fields(T, b1, b2, b3, start[c + 1] - start[c]);
+            if (slabs && r == 0u) cur[c] = slab_fields(T, b1, b2, b3, start[c + 1] - start[c]);
             skey[f] = (uint32_t)(c + lo);
             if (!GATHER) sval[f] = e;
             if (GATHER) {
@@ -515,10 +613,12 @@ __global__ __launch_bounds__(OT) void cell_sort_one_kernel(
             __syncthreads();
         }
     };
-    if (count <= (uint32_t)kOneList) order(ordE, ordK, true);
+    if (count <= (uint32_t)list) order(ordE, ordK, true);
     else order(tmpE + base, tmpK + base, false);
     __syncthreads();
-    for (int c = tid; c < own; c += OT) cs[c + lo] = table[c];
+    const uint32_t empty = T.empty();
+    for (int c = tid; c < own; c += OT)
+        cs[c + lo] = (base + start[c]) | (start[c] == start[c + 1] ? empty : slabs ? cur[c] : 0u);
     if (hi == m && tid == 0) cs[m] = (uint32_t)n;
 }
 
@@ -527,7 +627,7 @@ inline int cblocks(int64_t n) { return (int)((n + CT - 1) / CT); }
 }  // namespace
 
 bool cell_sort_one(const sph_ctx* c) {
-    return c->n <= kOneSort && c->sc.cs_cells <= kOneGroups * kOneCells;
+    return c->n <= kOneSort && c->sc.cs_cells <= kOneMost;
 }
 
 int64_t cell_scan_tiles(int64_t cells) { return (cells + CTILE - 1) / CTILE; }
@@ -548,11 +648,13 @@ hipError_t launch_cell_sort(sph_ctx* c, bool gather, hipStream_t s, bool counted
     c->sorted_keys = b.keyS[1];
     c->sorted_vals = b.valS[1];
     if (cell_sort_one(c)) {
-        const int per = std::max(1, (m + kOneGroups - 1) / kOneGroups);
-        const int groups = std::max(1, (m + per - 1) / per);
-        const size_t lds = sizeof(uint32_t) * ((size_t)3 * per + 1 + 4 * kOneList + heavy_words(n, gather && T.shift > 0));
+        const int shares = one_shares(n), most = kOneGroups - shares;
+        const int per = std::max(1, (m + most - 1) / most), ranges = std::max(1, (m + per - 1) / per);
+        const int groups = ranges + shares;
+        const size_t lds = sizeof(uint32_t) * (2 * (size_t)per + 1 + 2 * one_list(n) +
+                                               std::max(2 * one_list(n), heavy_words(n, gather && T.shift > 0)));
         (gather ? cell_sort_one_kernel<true> : cell_sort_one_kernel<false>)<<<groups, OT, lds, s>>>(
-            n, m, per, T, b.keyI, b.pidB, b.cs, b.keyS[1], b.valS[1], b.posB, b.velB, b.posA, b.velA, b.pidA, tmp,
+            n, m, per, ranges, T, b.keyI, b.pidB, b.cs, b.keyS[1], b.valS[1], b.posB, b.velB, b.posA, b.velA, b.pidA, tmp,
             rank);
         return hipGetLastError();
     }
