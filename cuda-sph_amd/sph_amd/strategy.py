@@ -90,19 +90,30 @@ class SPHStrategy:
 
     # -- reference entry point -----------------------------------------------------------
     def compute_next_state(self, old_state: SimulationState) -> SimulationState:
-        return self.advance(old_state, 1)
+        return self._advance(old_state, 1)
 
     def advance(self, state: SimulationState, nsteps: int) -> SimulationState:
         """nsteps steps with one upload and one download."""
+        return self._advance(state, int(nsteps))
+
+    def _advance(self, state: SimulationState, nsteps: int) -> SimulationState:
         self.old_state = state
-        if self.keep_terms:
+        if self.keep_terms or self._stages_replaced():
             self._initialize_computation()
-            self.ctx.step(int(nsteps))
+            self.ctx.step(nsteps)
             self._finalize_computation()
         else:
             # copies, steps and the finite check in one call, through page-locked memory
-            self._returned(self.ctx.advance_host(self._new_arrays(), int(nsteps)))
+            self._returned(self.ctx.advance_host(self._new_arrays(), nsteps))
         return self.new_state
+
+    def _stages_replaced(self) -> bool:
+        """Whether a subclass or this object has its own first or last stage, which one call for
+        the copies and the steps would pass over."""
+        for name in ("_initialize_computation", "_finalize_computation"):
+            if getattr(getattr(self, name), "__func__", None) is not getattr(SPHStrategy, name):
+                return True
+        return False
 
     def capture(self, nsteps: int) -> torch.cuda.CUDAGraph:
         """A HIP graph of nsteps steps of the resident state (recorded, not run).  The step
