@@ -85,6 +85,15 @@ __device__ __forceinline__ float group_sum(float v) {
     }));
 }
 
+// Between the stores to LDS of some lanes of a wavefront and the loads of others, and back: a
+// wavefront's LDS accesses are carried out in order, so nothing is waited for, but the compiler
+// has to keep them in it.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Raw buffer loads with 32-bit byte offsets: no 64-bit address arithmetic per access, and
 // an offset past num_records reads zero instead of faulting.  Word 3 of the descriptor is
 // the gfx9 value for untyped 32-bit-element buffers.
@@ -1048,9 +1057,9 @@ __device__ __forceinline__ PairSums naive_pair_sums_ordered(const StepConsts& C,
         buf[7u * kPitch + at] = vj.z - v.z;
     };
     auto add = [&](uint32_t count) {
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_order();
         for (uint32_t t = 0; t < count; ++t) acc += coef[t] * part[t];
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_order();
     };
     const uint32_t head = nn[i];
     const uint32_t cnt = head < kNoList ? min(head, (uint32_t)kListCap) : 0u;

@@ -365,7 +365,9 @@ __device__ __forceinline__ void density_particle(const StepConsts& G, const Step
         uint32_t kept = 0;  // terms not added yet
         auto add_terms = [&]() {
             // whole float4s: a term of zero adds nothing
+            static_assert(!ORDERED || L >= 4, "three lanes fill the last one up");
             if (l < 3u) terms[kept + l] = 0.0f;
+            wave_lds_order();
             for (uint32_t t = 0; t < kept; t += 4u) {
                 const float4 u = *reinterpret_cast<const float4*>(terms + t);
                 acc += u.x * u.x * u.x;
@@ -373,6 +375,7 @@ __device__ __forceinline__ void density_particle(const StepConsts& G, const Step
                 acc += u.z * u.z * u.z;
                 acc += u.w * u.w * u.w;
             }
+            wave_lds_order();
             kept = 0;
         };
         // one candidate per lane of the group, hits ranked by a ballot
@@ -406,6 +409,7 @@ __device__ __forceinline__ void density_particle(const StepConsts& G, const Step
         khi = group_fold<L>(khi, [](uint32_t a, uint32_t b) { return max(a, b); });
     }
     if (!ORDERED) acc = group_sum<L>(acc);
+    if constexpr (L > 1) wave_lds_order();
     const uint32_t staged = cnt < kCap ? cnt : kCap;
     // the staged slots as 32-bit words (two slots each), the group's lanes taking turns
     uint32_t* words = reinterpret_cast<uint32_t*>(nl);
@@ -779,7 +783,7 @@ __global__ __launch_bounds__(256) void voxel_density_group_kernel(StepConsts C, 
             }
             cnt = min(cnt + __popc(hits), kMaxNeighbours);
         }
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_order();
         float acc = 0.0f;
         for (int t0 = 0; t0 < cnt; t0 += 4) {  // a term of zero adds nothing
             const float4 t = *reinterpret_cast<const float4*>(&s_term[part][t0]);
@@ -900,7 +904,7 @@ __global__ __launch_bounds__(256) void voxel_force_group_kernel(
         buf[6u * kPitch + l] = self ? 0.0f : vj.y - v.y;
         buf[7u * kPitch + l] = self ? 0.0f : vj.z - v.z;
     }
-    __builtin_amdgcn_wave_barrier();
+    wave_lds_order();
     const uint32_t comp = l < 6u ? l : 5u;
     const float* const coef = buf + (comp < 3u ? 0u : kPitch);
     const float* const part = buf + (2u + comp) * kPitch;
