@@ -1123,11 +1123,19 @@ int ordered_lanes(const sph_ctx* c) {
 //                       59.4 / 88.5; dam break of 55,296 47.5 / 29.4, 96,256 36.0 / 33.8
 //     0.5 to 0.95       dam break of 66,048 169 / 48, 96,256 66 / 46, 131,072 75 / 68, 307,200
 //                       174.0 / 173.4
-//     less              24,576 375 / 35, 131,072 298 / 128, 307,200 733 / 411
+//     0.15 to 0.5       24,576 375 / 35, 131,072 298 / 128, 307,200 733 / 411
+// Far coarser voxels hold thousands of particles, whose candidates fill the lanes of both; one lane reads
+// each of them for the whole wavefront then.  ms per launch, box (30 and 105 neighbours), at h of
+//     0.1 edges         65,536 3.0 / 1.2 and 8.5 / 3.1, 131,072 4.9 / 2.7 and 11.5 / 8.8, 200,000 5.0 / 3.9 and
+//                       12.9 / 15.7, 307,200 7.8 / 6.9 and 14.6 / 20.0
+//     0.05              98,304 10.8 / 5.4 and 11.0 / 4.9, 131,072 17.3 / 16.2 and 22.7 / 14.5, 200,000 26.2 / 36.9
+//                       and 29.2 / 27.8
+//     0.02              65,536 6.9 / 4.3, 98,304 10.1 / 9.2, 131,072 13.4 / 16.1, 307,200 43.8 / 102.3
 bool voxel_groups(const sph_ctx* c) {
     const float edge = fmaxf(c->sc.cell[0], fmaxf(c->sc.cell[1], c->sc.cell[2]));
     const float h = c->sc.h;
-    return c->n <= (h >= 0.95f * edge ? 98304 : h >= 0.5f * edge ? 131072 : 307200);
+    const bool few = h >= 0.95f * edge || h < 0.04f * edge;
+    return c->n <= (few ? 98304 : h >= 0.5f * edge || h < 0.15f * edge ? 131072 : 307200);
 }
 
 // Up to this many particles the VOXEL force pass gives each 32 lanes.  us per launch, one lane / 32
