@@ -756,7 +756,9 @@ __global__ __launch_bounds__(256) void voxel_density_group_kernel(StepConsts C, 
         const int dx = (int)l / 9 - 1, dy = (int)l / 3 % 3 - 1, dz = (int)l % 3 - 1;
         const int nx = ref_coord(p.x, 0, C) + dx, ny = ref_coord(p.y, 1, C) + dy, nz = ref_coord(p.z, 2, C) + dz;
         uint32_t start = 0u, end = 0u;
-        if (l < 27u && nx >= 0 && nx < C.tdims[0] && ny >= 0 && ny < C.tdims[1] && nz >= 0 && nz < C.tdims[2]) {
+        // a NaN or infinite particle has no neighbours; looking for them among all such particles,
+        // which share a voxel, took the group 102 ms with 307,200 of them and one lane 46
+        if (finite3(p.x, p.y, p.z) && l < 27u && nx >= 0 && nx < C.tdims[0] && ny >= 0 && ny < C.tdims[1] && nz >= 0 && nz < C.tdims[2]) {
             const float e2 = voxel_slab2(p.x, nx, C.cell[0]) + voxel_slab2(p.y, ny, C.cell[1]) +
                              voxel_slab2(p.z, nz, C.cell[2]);
             if (!(skip_ok && e2 > C.h_search * C.h_search)) {

@@ -23,7 +23,7 @@ def strategy(n, h, edges, gpu):
 
 # with one particle more the density pass has one lane per particle; h of 0.02 edges, or every
 # particle NaN (all of them in one voxel, no pair within h)
-@pytest.mark.parametrize("form", ["coarse"])
+@pytest.mark.parametrize("form", ["coarse", "nan"])
 def test_a_crowd_costs_no_more_than_with_one_lane(gpu, form):
     def density_ms(n):
         h = 0.4 * (30 / (4.0 / 3.0 * np.pi * n)) ** (1.0 / 3.0)
