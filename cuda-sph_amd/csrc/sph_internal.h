@@ -109,6 +109,8 @@ struct StepConsts {
     int lanes;
     int lane_shift;
     int tfirst;
+    // totals: whether the batched passes deal their workgroups out to the XCDs in chunks
+    int spread;
     // NAIVE grid keys: each cell is cut into S = 1 << slab_shift slabs along x (1: not cut).
     // A key carries its particle's slab in bits kSlabKeyShift.. (the cell below them); the
     // fused step's sort orders the particles of a cell by (slab, id), and the entry of an

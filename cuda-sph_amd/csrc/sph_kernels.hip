@@ -491,7 +491,8 @@ __global__ __launch_bounds__(kDensityThreads) void naive_density_batch_kernel(St
                                                                                ListEntry* __restrict__ nl,
                                                                                uint32_t* __restrict__ nn) {
     __shared__ __align__(16) DensityList s_stage[kDensityThreads / 64];
-    const uint32_t gt = (uint32_t)xcd_chunk_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+    const int tile = G.spread ? xcd_chunk_tile(blockIdx.x, gridDim.x) : xcd_tile(blockIdx.x, gridDim.x);
+    const uint32_t gt = (uint32_t)tile * blockDim.x + threadIdx.x;
     const BatchLane t = batch_lane(G, gt);
     if (t.i < 0) return;
     const StepConsts& C = G.inst_table[t.b];
@@ -583,7 +584,8 @@ __global__ __launch_bounds__(256) void naive_force_batch_kernel(
     const uint32_t* __restrict__ nn, float4* __restrict__ posOut, float4* __restrict__ velOut,
     uint32_t* __restrict__ pidOut, uint32_t* __restrict__ keyI, uint32_t* __restrict__ valI,
     float4* __restrict__ dbgP, float4* __restrict__ dbgV, float4* __restrict__ dbgF, uint32_t* __restrict__ flags) {
-    const uint32_t gt = (uint32_t)xcd_chunk_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+    const int tile = G.spread ? xcd_chunk_tile(blockIdx.x, gridDim.x) : xcd_tile(blockIdx.x, gridDim.x);
+    const uint32_t gt = (uint32_t)tile * blockDim.x + threadIdx.x;
     const BatchLane t = batch_lane(G, gt);
     if (t.i < 0) return;
     const StepConsts& C = G.inst_table[t.b];
