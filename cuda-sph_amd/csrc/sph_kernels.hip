@@ -480,10 +480,21 @@ __device__ __forceinline__ BatchLane batch_lane(const StepConsts& G, uint32_t gt
     return r;
 }
 
-// TOP, 16 or 64, is the largest group that the kernel has code for: the path of 32 lanes over rows
-// laid end to end costs the others 4% where it stands beside them (64 boxes of 2,048 to 65,536
-// particles at up to 16 lanes, 4 steps, before these shared rows: 5.98 ms, 5.74 without it).  A larger group than TOP, which
-// a graph captured before the lanes were set can meet, works with its first TOP lanes.
+// f with the group size `lanes` as a compile-time constant, among those up to TOP that a batched kernel
+// has code for.  A larger group, which a graph captured before the lanes were set can meet, works
+// with its first TOP lanes.
+template <int TOP, int L = 1, typename F>
+__device__ __forceinline__ void with_lanes(const BatchLane& t, F&& f) {
+    if constexpr (L < TOP) {
+        if (t.lanes > L) return with_lanes<TOP, 2 * L>(t, f);
+    }
+    if (t.l < (uint32_t)L) f(std::integral_constant<int, L>{});
+}
+
+// TOP is 1, 8, 16 or 64: the code of larger groups costs the smaller ones registers and time where it
+// stands beside them.  That of 32 lanes over rows laid end to end: 64 boxes of 2,048 to 65,536
+// particles at up to 16 lanes, 4 steps, before these shared rows, 5.98 ms, 5.74 without it.  That of
+// the others beside one lane: 8 of 60,000 particles 180 us per step, 166 without it.
 template <int TOP>
 __global__ __launch_bounds__(kDensityThreads) void naive_density_batch_kernel(StepConsts G, float4* pos, float4* vel,
                                                                                const uint32_t* __restrict__ cs,
@@ -500,22 +511,10 @@ __global__ __launch_bounds__(kDensityThreads) void naive_density_batch_kernel(St
     const uint32_t gbase = lane & ~(uint32_t)(t.lanes - 1);
     ListEntry* const base = s_stage[threadIdx.x >> 6];
     const uint32_t p = lane >> C.lane_shift;  // the particle's place in the wavefront's band
-    switch (t.lanes) {
-        case 1: density_particle<1>(G, C, t.i, 0u, StageBand<1>{base, p}, gbase, pos, vel, cs, rhoA, nl, nn); break;
-        case 2: density_particle<2>(G, C, t.i, t.l, StageBand<2>{base, p}, gbase, pos, vel, cs, rhoA, nl, nn); break;
-        case 4: density_particle<4>(G, C, t.i, t.l, StageBand<4>{base, p}, gbase, pos, vel, cs, rhoA, nl, nn); break;
-        case 8: density_particle<8>(G, C, t.i, t.l, StageBand<8>{base, p}, gbase, pos, vel, cs, rhoA, nl, nn); break;
-        case 16: density_particle<16>(G, C, t.i, t.l, StageBand<16>{base, p}, gbase, pos, vel, cs, rhoA, nl, nn); break;
-        case 32:
-            if constexpr (TOP > 32) {
-                density_particle<32>(G, C, t.i, t.l, StageBand<32>{base, p}, gbase, pos, vel, cs, rhoA, nl, nn);
-                break;
-            }
-            [[fallthrough]];
-        default:
-            if (t.l < (uint32_t)TOP)
-                density_particle<TOP>(G, C, t.i, t.l, StageBand<TOP>{base, p}, gbase, pos, vel, cs, rhoA, nl, nn);
-    }
+    with_lanes<TOP>(t, [&](auto size) {
+        constexpr int L = decltype(size)::value;
+        density_particle<L>(G, C, t.i, t.l, StageBand<L>{base, p}, gbase, pos, vel, cs, rhoA, nl, nn);
+    });
 }
 
 // Force pass (naive_kernels.py:24-80) fused with integration and collision: each lane
@@ -592,21 +591,9 @@ __global__ __launch_bounds__(256) void naive_force_batch_kernel(
     const int i = t.i;
     const float4 p = pos[i], v = vel[i];
     PairSums S;
-    switch (t.lanes) {
-        case 1: S = naive_pair_sums_lanes<1>(C, i, 0u, G.n, p, v, pos, vel, cs, nl, nn); break;
-        case 2: S = naive_pair_sums_lanes<2>(C, i, t.l, G.n, p, v, pos, vel, cs, nl, nn); break;
-        case 4: S = naive_pair_sums_lanes<4>(C, i, t.l, G.n, p, v, pos, vel, cs, nl, nn); break;
-        case 8: S = naive_pair_sums_lanes<8>(C, i, t.l, G.n, p, v, pos, vel, cs, nl, nn); break;
-        case 16: S = naive_pair_sums_lanes<16>(C, i, t.l, G.n, p, v, pos, vel, cs, nl, nn); break;
-        case 32:
-            if constexpr (TOP > 32) {
-                S = naive_pair_sums_lanes<32>(C, i, t.l, G.n, p, v, pos, vel, cs, nl, nn);
-                break;
-            }
-            [[fallthrough]];
-        default:
-            if (t.l < (uint32_t)TOP) S = naive_pair_sums_lanes<TOP>(C, i, t.l, G.n, p, v, pos, vel, cs, nl, nn);
-    }
+    with_lanes<TOP>(t, [&](auto size) {
+        S = naive_pair_sums_lanes<decltype(size)::value>(C, i, t.l, G.n, p, v, pos, vel, cs, nl, nn);
+    });
     if (t.l != 0) return;
     const float ps = 0.5f * C.mass * C.grad_c;
     const float vs = C.mass * C.visc * C.lap_c;
@@ -1198,12 +1185,12 @@ void launch_density_lanes(sph_ctx* c, hipStream_t s) {
     naive_density_kernel<L, FAR, ORDERED, MASKED, AHEAD><<<blocks_for(c->n * L, bs), bs, 0, s>>>(c->sc, b.posA, b.velA, b.cs, b.rhoA, b.nl, b.nn);
 }
 
-// Most lanes of an instance: up to 16, the batch's passes leave out what 32 and 64 lanes need
-// (naive_density_batch_kernel).
-int batch_top_lanes(const sph_ctx* c) {
+// The batched kernel, of those for groups of up to 1, 8, 16 and 64 lanes, that serves all instances.
+template <typename K>
+K batch_kernel(const sph_ctx* c, K one, K eight, K sixteen, K all) {
     int top = 1;
     for (const StepConsts& S : c->inst) top = max(top, S.lanes);
-    return top;
+    return top == 1 ? one : top <= 8 ? eight : top <= 16 ? sixteen : all;
 }
 
 hipError_t launch_density(sph_ctx* c, hipStream_t s) {
@@ -1222,9 +1209,9 @@ hipError_t launch_density(sph_ctx* c, hipStream_t s) {
     }
     if (!c->inst.empty()) {
         const Buffers& b = c->b;
-        const auto kernel = batch_top_lanes(c) > 16 ? naive_density_batch_kernel<64> : naive_density_batch_kernel<16>;
-        kernel<<<blocks_for(c->sc.tfirst, bs), bs, 0, s>>>(c->sc, b.posA, b.velA, b.cs, b.rhoA,
-                                                                              b.nl, b.nn);
+        const auto kernel = batch_kernel(c, naive_density_batch_kernel<1>, naive_density_batch_kernel<8>,
+                                         naive_density_batch_kernel<16>, naive_density_batch_kernel<64>);
+        kernel<<<blocks_for(c->sc.tfirst, bs), bs, 0, s>>>(c->sc, b.posA, b.velA, b.cs, b.rhoA, b.nl, b.nn);
         return hipGetLastError();
     }
     switch (c->lanes) {
@@ -1280,7 +1267,8 @@ void launch_force_mode(sph_ctx* c, hipStream_t s, bool count) {
         return;
     }
     if (!c->inst.empty()) {  // batched instances have box walls
-        const auto kernel = batch_top_lanes(c) > 16 ? naive_force_batch_kernel<64> : naive_force_batch_kernel<16>;
+        const auto kernel = batch_kernel(c, naive_force_batch_kernel<1>, naive_force_batch_kernel<8>,
+                                         naive_force_batch_kernel<16>, naive_force_batch_kernel<64>);
         kernel<<<blocks_for(c->sc.tfirst, bs), bs, 0, s>>>(
             c->sc, c->b.posA, c->b.velA, c->b.pidA, c->b.rhoA, c->b.cs, c->b.nl, c->b.nn, c->b.posB, c->b.velB,
             c->b.pidB, c->b.keyI, c->b.valI, dP, dV, dF, c->b.flags);
