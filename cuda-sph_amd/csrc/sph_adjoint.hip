@@ -100,7 +100,7 @@ __device__ __forceinline__ void walk_neighbours_lanes(const StepConsts& C, int i
                 const uint32_t last = list_decode(nl[list_at(C.n, i, kListCap - 1)], i);
                 tail = ListTail(last, pos[last], C);
             }
-            for_each_batch<L>(
+            for_each_batch<L, kScanAtOnce<L>>(
                 p.x, p.y, p.z, C, rcs, make_rsrc(pos, (uint32_t)C.n * 16u), l, [](uint32_t, uint32_t) {},
                 [&](uint32_t k, float4 q, bool valid) {
                     const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;

@@ -414,9 +414,11 @@ struct RowWindows {
 // not wait for each batch in turn.  With 32 lanes, which rows rarely fill, the rows of one pass
 // over t are laid end to end and taken L at a time across their bounds; a lane finds its row from
 // the places where rows start, without LDS memory (20-step gradients of 16,384 particles
-// 1.575 -> 1.51 ms; with 16 lanes it lost 6% over the 64-box batch).  Without AHEAD each row is
-// taken by itself and nothing is loaded before it is needed.  From the tail's start on, without the candidates before the tail's first.  rows(k0, k1) gets the lane's own row ranges.
-template <int L, bool AHEAD = true, typename RowF, typename F>
+// 1.575 -> 1.51 ms; with 16 lanes it lost 6% over the 64-box batch).
+// AT_ONCE > 0: each row is taken by itself, AT_ONCE batches of it loaded together.
+// From the tail's start on, without the candidates before the tail's first.  rows(k0, k1) gets the
+// lane's own row ranges.
+template <int L, int AT_ONCE = 0, typename RowF, typename F>
 __device__ __forceinline__ void for_each_batch(float px, float py, float pz, const StepConsts& C,
                                                __amdgpu_buffer_rsrc_t rcs, __amdgpu_buffer_rsrc_t rpos, uint32_t l,
                                                RowF&& rows, F&& f, ListTail tail = ListTail()) {
@@ -458,12 +460,27 @@ __device__ __forceinline__ void for_each_batch(float px, float py, float pz, con
             }
             continue;
         }
-        if constexpr (!AHEAD) {
+        if constexpr (AT_ONCE == 1) {
             for (int j = 0; j < min(L, npairs - t0); ++j) {
                 const uint32_t k0 = __shfl(a0, gbase + j), k1 = __shfl(a1, gbase + j);
                 for (uint32_t b = k0; b < k1; b += L) {
                     const uint32_t k = b + l;
                     f(k, ld_f4(rpos, k * 16u), k < k1);
+                }
+            }
+            continue;
+        }
+        if constexpr (AT_ONCE > 1) {
+            while (left != 0ull) {
+                const int j = gbase + __ffsll((unsigned long long)left) - 1;
+                left &= left - 1ull;
+                const uint32_t k0 = __shfl(a0, j) + l, k1 = __shfl(a1, j);
+                for (uint32_t k = k0; k - l < k1; k += (uint32_t)(AT_ONCE * L)) {
+                    float4 q[AT_ONCE];
+#pragma unroll
+                    for (int u = 0; u < AT_ONCE; ++u) q[u] = ld_f4(rpos, (k + (uint32_t)(u * L)) * 16u);
+#pragma unroll
+                    for (int u = 0; u < AT_ONCE; ++u) f(k + (uint32_t)(u * L), q[u], k + (uint32_t)(u * L) < k1);
                 }
             }
             continue;
@@ -494,6 +511,15 @@ __device__ __forceinline__ void for_each_batch(float px, float py, float pz, con
         }
     }
 }
+
+// The batches that a scan of a particle's candidates in place of its list, by the force pass and the
+// pullbacks, takes at once (for_each_batch): it meets rows of many batches, and few lanes wait on each
+// load.  Step and 4-step gradients of a box with 300 and 250 neighbours, looking one batch ahead and
+// with this, 2 lanes of 4,099 particles 413 -> 357 us and 8,192 4.11 -> 3.44 ms, 4 lanes 189 -> 170 and
+// 2.10 -> 1.75, 8 lanes 102 -> 95 and 1.20 -> 1.09 (as many as one per lane before: 396 and 3.74, 191
+// and 2.00, 108 and 1.22).
+template <int L>
+constexpr int kScanAtOnce = L <= 4 ? 3 : L == 8 ? 2 : 0;
 
 __device__ __forceinline__ float lane_of(float v, int lane) {
     return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(v), lane));
@@ -999,7 +1025,7 @@ __device__ __forceinline__ PairSums naive_pair_sums_lanes(const StepConsts& C, i
                 const uint32_t last = list_decode(nl[list_at(n, i, kListCap - 1)], i);
                 tail = ListTail(last, ld_f4(rpos, last * 16u), C);
             }
-            for_each_batch<L>(
+            for_each_batch<L, kScanAtOnce<L>>(
                 p.x, p.y, p.z, C, rcs, rpos, l, [](uint32_t, uint32_t) {},
                 [&](uint32_t k, float4 q, bool valid) {
                     const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;

@@ -379,7 +379,7 @@ __device__ __forceinline__ void density_particle(const StepConsts& G, const Step
             kept = 0;
         };
         // one candidate per lane of the group, hits ranked by a ballot
-        for_each_batch<L, AHEAD>(
+        for_each_batch<L, AHEAD ? 0 : 1>(
             p.x, p.y, p.z, C, rcs, rpos, l,
             [&](uint32_t k0, uint32_t k1) {
                 klo = min(klo, k0);
