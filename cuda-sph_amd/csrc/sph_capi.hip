@@ -886,17 +886,17 @@ int sph_advance_host(sph_ctx* c, int32_t nsteps, const double* pos, const double
     double* const dpos = (double*)(dev + kStagingHead);
     double* const dvel = dpos + 3 * n;
     HostCopy copy;
-    if ((rc = copy.open(pinned, pinned_bytes, n, s))) return rc;
-    if (pos) {
-        if ((rc = copy.to_device(dev, pos, vel))) return rc;
-        if ((rc = sph_upload_state(c, dpos, dvel, stream))) return rc;
-    }
-    if ((rc = run_steps(c, s, nsteps))) return rc;
     const bool check = c->check_finite && nsteps > 0;
-    if ((rc = hip_check(sph::launch_download_f64(c, dpos, dvel, dvel + 3 * n, nullptr, s, check ? (uint32_t*)dev : nullptr),
-                        "download")))
-        return rc;
-    return copy.to_host(dev, pos_out, vel_out, rho_out, check);
+    rc = copy.open(pinned, pinned_bytes, n, s);
+    if (rc == SPH_OK && pos) rc = copy.to_device(dev, pos, vel);
+    if (rc == SPH_OK && pos) rc = sph_upload_state(c, dpos, dvel, stream);
+    if (rc == SPH_OK) rc = run_steps(c, s, nsteps);
+    if (rc == SPH_OK)
+        rc = hip_check(sph::launch_download_f64(c, dpos, dvel, dvel + 3 * n, nullptr, s, check ? (uint32_t*)dev : nullptr),
+                       "download");
+    if (rc == SPH_OK) return copy.to_host(dev, pos_out, vel_out, rho_out, check);
+    (void)hipStreamSynchronize(s);  // copies already enqueued use the caller's memory
+    return rc;
 }
 
 int64_t sph_buffer_elems(const sph_ctx* c, int32_t which) {
