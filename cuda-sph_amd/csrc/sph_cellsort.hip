@@ -608,8 +608,8 @@ __global__ __launch_bounds__(OT) void cell_sort_one_kernel(
                 return r + (uint32_t)__popc(bits[word] & ((1u << (x & 31u)) - 1u));
             };
             for (uint32_t t = a + tid; t < b; t += OT)
-                put(t, c, before(place_of(K[t])), slabs ? before((uint32_t)n) : 0u, slabs ? before(2u * (uint32_t)n) : 0u,
-                    slabs ? before(3u * (uint32_t)n) : 0u);
+                put(t, c, before(place_of(K[t])), slabs ? before((uint32_t)n) : 0u,
+                    slabs ? before(2u * (uint32_t)n) : 0u, slabs ? before(3u * (uint32_t)n) : 0u);
             __syncthreads();
         }
     };
@@ -654,8 +654,8 @@ hipError_t launch_cell_sort(sph_ctx* c, bool gather, hipStream_t s, bool counted
         const size_t lds = sizeof(uint32_t) * (2 * (size_t)per + 1 + 2 * one_list(n) +
                                                std::max(2 * one_list(n), heavy_words(n, gather && T.shift > 0)));
         (gather ? cell_sort_one_kernel<true> : cell_sort_one_kernel<false>)<<<groups, OT, lds, s>>>(
-            n, m, per, ranges, T, b.keyI, b.pidB, b.cs, b.keyS[1], b.valS[1], b.posB, b.velB, b.posA, b.velA, b.pidA, tmp,
-            rank);
+            n, m, per, ranges, T, b.keyI, b.pidB, b.cs, b.keyS[1], b.valS[1], b.posB, b.velB, b.posA, b.velA, b.pidA,
+            tmp, rank);
         return hipGetLastError();
     }
     const bool summed = counted && tile_sums_in_force(c);

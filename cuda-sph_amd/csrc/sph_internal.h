@@ -199,7 +199,7 @@ struct sph_ctx {
     int pass_bits[4];
     int num_tiles;
     int density_block, force_block;
-    int lanes;               // NAIVE formulation: lanes of a wavefront per particle in density / force (1..16)
+    int lanes;               // NAIVE formulation: lanes of a wavefront per particle in density / force (1..64)
     int keep_terms;
     int check_finite;        // SPH_FLAG_CHECK_FINITE: sph_step reads the non-finite count
     int adjoint;             // SPH_FLAG_ADJOINT: reverse-mode buffers are part of the workspace

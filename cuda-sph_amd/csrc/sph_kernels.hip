@@ -268,11 +268,12 @@ constexpr uint32_t kOrderedTerms = 128;
 // ballot ranks them), so the neighbour list is the one a single lane builds, and the density
 // is summed per lane, then across the group.  G holds the totals (particle count, cell
 // table length), C the particle's own instance; band is the particle's place in its
-// wavefront's LDS staging band
-// (unique in the workgroup), gbase its group's first lane in the wavefront.  MASKED (L = 1): three
-// candidates at a time.  FAR (L = 1): lists beyond the int16 window too (kSeqList).  ORDERED (L > 1): the density is summed over the hits
-// in list order, as one lane sums it, to the same bits: the group keeps the hits' terms in terms
-// (kOrderedTerms words of LDS) and adds them up from there.  AHEAD (L > 1): see for_each_batch.
+// wavefront's LDS staging band (unique in the workgroup), gbase its group's first lane in the
+// wavefront.  MASKED (L = 1): three candidates at a time.  FAR (L = 1): lists beyond the int16
+// window too (kSeqList).  ORDERED (L > 1): the density is summed over the hits in list order, as
+// one lane sums it, to the same bits: the group keeps the hits' terms in terms (kOrderedTerms
+// words of LDS) and adds them up from there.  AHEAD (L > 1): candidates are loaded a batch ahead
+// (for_each_batch).
 template <int L, bool FAR = false, bool ORDERED = false, bool MASKED = false, bool AHEAD = true>
 __device__ __forceinline__ void density_particle(const StepConsts& G, const StepConsts& C, int i, uint32_t l,
                                                  StageBand<L> band, uint32_t gbase, float4* pos, float4* vel,
@@ -285,7 +286,9 @@ __device__ __forceinline__ void density_particle(const StepConsts& G, const Step
     const float4 p = pos[i];
     const size_t stride = (size_t)G.n;
     if constexpr (kSharesRows<L> && !ORDERED) {
-        if (__ballot(crowded(C, p, rcs)) == ~0ull && shared_density<L>(C, i, l, p, rpos, rcs, pos, vel, rhoA, nn)) return;
+        if (__ballot(crowded(C, p, rcs)) == ~0ull &&
+            shared_density<L>(C, i, l, p, rpos, rcs, pos, vel, rhoA, nn))
+            return;
     }
     float acc = 0.0f;
     uint32_t cnt = 0;
@@ -446,8 +449,8 @@ __global__ __launch_bounds__(kDensityThreads) void naive_density_kernel(StepCons
     const uint32_t lane = threadIdx.x & 63u;
     const StageBand<L> band{s_stage[threadIdx.x >> 6], lane / L};
     __shared__ __align__(16) float s_terms[ORDERED ? kDensityThreads / L : 1][ORDERED ? kOrderedTerms : 1];
-    density_particle<L, FAR, ORDERED, MASKED, AHEAD>(G, G, i, gt & (L - 1), band, lane & ~(uint32_t)(L - 1), pos, vel, cs, rhoA, nl, nn,
-                                      s_terms[ORDERED ? threadIdx.x / L : 0]);
+    density_particle<L, FAR, ORDERED, MASKED, AHEAD>(G, G, i, gt & (L - 1), band, lane & ~(uint32_t)(L - 1), pos,
+                                                     vel, cs, rhoA, nl, nn, s_terms[ORDERED ? threadIdx.x / L : 0]);
 }
 
 // Batched form: each instance has its own lanes per particle and its own thread range, which
@@ -480,9 +483,10 @@ __device__ __forceinline__ BatchLane batch_lane(const StepConsts& G, uint32_t gt
     return r;
 }
 
-// f with the group size `lanes` as a compile-time constant, among those up to TOP that a batched kernel
-// has code for.  A larger group, which a graph captured before the lanes were set can meet, works
-// with its first TOP lanes.
+// f with the group's size as a compile-time constant, among those up to TOP that a batched kernel has
+// code for.  A larger group, which only a graph recorded before the lanes were set can meet, would
+// work with its first TOP lanes (the graph has to be recorded again: its launch may not reach
+// all groups).
 template <int TOP, int L = 1, typename F>
 __device__ __forceinline__ void with_lanes(const BatchLane& t, F&& f) {
     if constexpr (L < TOP) {
@@ -520,8 +524,8 @@ __global__ __launch_bounds__(kDensityThreads) void naive_density_batch_kernel(St
 // Force pass (naive_kernels.py:24-80) fused with integration and collision: each lane
 // walks its particle's neighbour list (one coalesced load per slot, kForceUnroll slots and
 // their gathers in flight); a particle with more neighbours than list slots scans its list's
-// tail or all of its candidates instead.  With L lanes per particle the group splits the list (or the rescan)
-// and lane 0 finishes the particle.  MODE selects the wall collision at compile time.
+// tail or all of its candidates instead.  With L lanes per particle the group splits the list (or
+// the rescan) and lane 0 finishes the particle.  MODE selects the wall collision at compile time.
 template <int MODE, int L = 1, bool COUNT = false, bool ORDERED = false>
 __global__ __launch_bounds__(256) void naive_force_kernel(
     StepConsts G, const float4* __restrict__ pos, const float4* __restrict__ vel, const uint32_t* __restrict__ pidA,
@@ -747,7 +751,8 @@ __global__ __launch_bounds__(256) void voxel_density_group_kernel(StepConsts C, 
         uint32_t start = 0u, end = 0u;
         // a NaN or infinite particle has no neighbours; looking for them among all such particles,
         // which share a voxel, took the group 102 ms with 307,200 of them and one lane 46
-        if (finite3(p.x, p.y, p.z) && l < 27u && nx >= 0 && nx < C.tdims[0] && ny >= 0 && ny < C.tdims[1] && nz >= 0 && nz < C.tdims[2]) {
+        if (finite3(p.x, p.y, p.z) && l < 27u && nx >= 0 && nx < C.tdims[0] && ny >= 0 && ny < C.tdims[1] &&
+            nz >= 0 && nz < C.tdims[2]) {
             const float e2 = voxel_slab2(p.x, nx, C.cell[0]) + voxel_slab2(p.y, ny, C.cell[1]) +
                              voxel_slab2(p.z, nz, C.cell[2]);
             if (!(skip_ok && e2 > C.h_search * C.h_search)) {
@@ -792,7 +797,8 @@ __global__ __launch_bounds__(256) void voxel_density_group_kernel(StepConsts C, 
     __syncthreads();
     // thread t of the block: slot t / parts of particle t % parts
     const int slot = (int)threadIdx.x / parts, mine = (int)threadIdx.x % parts;
-    if (first + mine < C.n && slot < s_count[mine]) nbr[(size_t)(1 + slot) * (size_t)C.n + first + mine] = s_list[mine][slot];
+    if (first + mine < C.n && slot < s_count[mine])
+        nbr[(size_t)(1 + slot) * (size_t)C.n + first + mine] = s_list[mine][slot];
 }
 
 // Coefficients of one pair's pressure term (of x_i - x_j) and viscosity term (of v_j - v_i).
@@ -1102,6 +1108,11 @@ constexpr int64_t kMaskedParticles = 307200;
 //    65,536             41 / 11      30 / 14      30 / 17
 //    98,304             49 / 14      40 / 17      39 / 22
 //   131,072             45 / 16      56 / 22      78 / 30
+// The two passes share a limit, though from 65,536 particles on the force pass of sparse ones is
+// slower by groups (and they need the sort's tile sums counted apart): the host cannot tell
+// them from dense ones, whose force pass gains.  us per step, one lane / groups, with 30, 105 and
+// 300 neighbours: 65,536 particles 74 / 56, 283 / 116, 810 / 432, 98,304 85 / 76, 352 / 163,
+// 1,023 / 621.
 int ordered_lanes(const sph_ctx* c) {
     if (c->lanes != 1 || !c->inst.empty() || c->sc.formulation != SPH_FORM_NAIVE) return 1;
     return c->n <= 24576 ? 16 : c->n <= 98304 ? 8 : 1;
@@ -1141,21 +1152,24 @@ hipError_t launch_fill_u32(uint32_t* p, uint32_t v, int64_t n, hipStream_t s) {
 
 hipError_t launch_upload_f64(sph_ctx* c, const double* pos, const double* vel, hipStream_t s) {
     if (c->n > 0)
-        (c->sc.n_inst > 1 ? upload_f64_kernel<true> : upload_f64_kernel<false>)<<<blocks_for(c->n, 256), 256, 0, s>>>(c->sc, pos, vel, c->b.posB, c->b.velB, c->b.pidB,
-                                                                  c->b.keyI, c->b.valI, c->b.flags);
+        (c->sc.n_inst > 1 ? upload_f64_kernel<true> : upload_f64_kernel<false>)
+            <<<blocks_for(c->n, 256), 256, 0, s>>>(c->sc, pos, vel, c->b.posB, c->b.velB, c->b.pidB, c->b.keyI,
+                                                   c->b.valI, c->b.flags);
     return hipGetLastError();
 }
 
 hipError_t launch_upload_f32(sph_ctx* c, const float* x, const float* y, const float* z, const float* vx,
                              const float* vy, const float* vz, hipStream_t s) {
     if (c->n > 0)
-        (c->sc.n_inst > 1 ? upload_f32_kernel<true> : upload_f32_kernel<false>)<<<blocks_for(c->n, 256), 256, 0, s>>>(c->sc, x, y, z, vx, vy, vz, c->b.posB, c->b.velB,
-                                                                  c->b.pidB, c->b.keyI, c->b.valI, c->b.flags);
+        (c->sc.n_inst > 1 ? upload_f32_kernel<true> : upload_f32_kernel<false>)
+            <<<blocks_for(c->n, 256), 256, 0, s>>>(c->sc, x, y, z, vx, vy, vz, c->b.posB, c->b.velB, c->b.pidB,
+                                                   c->b.keyI, c->b.valI, c->b.flags);
     return hipGetLastError();
 }
 
 hipError_t launch_cell_table(sph_ctx* c, hipStream_t s) {
-    cell_table_kernel<<<blocks_for(c->n + 1, 256) + table_tile_blocks(c->sc), 256, 0, s>>>(c->sc, c->sorted_keys, c->b.cs);
+    const int blocks = blocks_for(c->n + 1, 256) + table_tile_blocks(c->sc);
+    cell_table_kernel<<<blocks, 256, 0, s>>>(c->sc, c->sorted_keys, c->b.cs);
     return hipGetLastError();
 }
 
@@ -1174,15 +1188,17 @@ hipError_t launch_rekey(sph_ctx* c, hipStream_t s) {
 // Up to this many threads groups of 2 and 4 lanes load a batch of candidates ahead (for_each_batch);
 // they take many batches per row, and with more wavefronts to hide the loads the bookkeeping
 // costs more.  us per launch, ahead / not: box of 65,537 particles at 4 lanes 24.6 / 25.8, 80,000
-// at 2 40.3 / 42.2, dam break of 42,000 at 4 19.8 / 23.8; of 137,500 at 2 42.0 / 38.1, 112,500 at 4
-// 32.4 / 28.0, 211,420 at 2 51.5 / 44.0.  Batches always look ahead (the 64 boxes 508 / 527).
+// at 2 40.3 / 42.2, dam break of 42,000 at 4 19.8 / 23.8, of 63,000 at 4 2% the other way; of 137,500
+// at 2 42.0 / 38.1, 112,500 at 4 32.4 / 28.0, 211,420 at 2 51.5 / 44.0.  Batches always look ahead
+// (the 64 boxes 508 / 527).
 constexpr int64_t kAheadThreads = 270000;
 
 template <int L, bool FAR = false, bool ORDERED = false, bool MASKED = false, bool AHEAD = true>
 void launch_density_lanes(sph_ctx* c, hipStream_t s) {
     const int bs = c->density_block;
     const Buffers& b = c->b;
-    naive_density_kernel<L, FAR, ORDERED, MASKED, AHEAD><<<blocks_for(c->n * L, bs), bs, 0, s>>>(c->sc, b.posA, b.velA, b.cs, b.rhoA, b.nl, b.nn);
+    naive_density_kernel<L, FAR, ORDERED, MASKED, AHEAD>
+        <<<blocks_for(c->n * L, bs), bs, 0, s>>>(c->sc, b.posA, b.velA, b.cs, b.rhoA, b.nl, b.nn);
 }
 
 // The batched kernel, of those for groups of up to 1, 8, 16 and 64 lanes, that serves all instances.

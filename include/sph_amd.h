@@ -169,8 +169,9 @@ int sph_download_state_f32(sph_ctx* ctx, float* dev_x, float* dev_y, float* dev_
  * float64, written when the call succeeds (also not when it returns SPH_E_NONFINITE; the
  * check is sph_step's).  dev_staging: device memory of at least sph_host_staging_bytes
  * bytes (256-byte aligned); pinned: page-locked host memory of pinned_bytes bytes, at least
- * 4,096 (256-byte aligned), through which the copies go, in two halves by turns where it is smaller than
- * the state.  Waits for the stream; not under graph capture. */
+ * 4,096 (256-byte aligned), through which the copies go, in two halves by turns where it is
+ * smaller than the state.  Waits for the stream, also when it fails on the way; not under
+ * graph capture. */
 size_t sph_host_staging_bytes(const sph_ctx* ctx);
 int sph_advance_host(sph_ctx* ctx, int32_t nsteps, const double* pos, const double* vel, double* pos_out,
                      double* vel_out, double* rho_out, void* dev_staging, size_t dev_bytes, void* pinned,
@@ -240,8 +241,7 @@ int sph_set_launch(sph_ctx* ctx, int32_t density_block, int32_t force_block);
  * many neighbours each) get that many times the parallelism.  The neighbour lists are the
  * same for every value; sums are added in a different order (FP32 rounding only).  With 1, a
  * plain context of few particles still shares each among several lanes, which add its sums in
- * one lane's order, to the same bits.  The
- * reference launches one thread per particle (thread_layout.py:27-33).  On a batched
+ * one lane's order, to the same bits.  The reference launches one thread per particle (thread_layout.py:27-33).  On a batched
  * context every instance gets `lanes`. */
 int sph_set_lanes(sph_ctx* ctx, int32_t lanes);
 
@@ -260,7 +260,9 @@ int sph_set_slabs(sph_ctx* ctx, int32_t enable, void* stream);
  * 1, 2, 4, 8, 16, 32 or 64), so that instances with many neighbours per particle get more lanes and
  * sparse ones fewer.  Each instance computes what a plain context with its lane count
  * computes.  The instance table is re-uploaded on `stream` (synchronised) when the workspace
- * is bound.  No counterpart in the reference, which advances one simulation per process. */
+ * is bound.  HIP graphs of sph_step recorded before the call (or sph_set_lanes on a batched
+ * context) keep the launches of the previous lanes, which may leave particles of the new
+ * ones unstepped: record them again.  No counterpart in the reference, which advances one simulation per process. */
 int sph_set_batch_lanes(sph_ctx* ctx, const int32_t* lanes, int32_t count, void* stream);
 
 /* Replaces the physics constants of a plain context between steps (the reference freezes
