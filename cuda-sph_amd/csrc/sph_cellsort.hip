@@ -384,7 +384,8 @@ __device__ __forceinline__ void one_share(const uint32_t* hist, int ranges, int 
     }
 }
 
-template <bool GATHER>
+// SHARED: one_shares(n) > 0.
+template <bool GATHER, bool SHARED>
 __global__ __launch_bounds__(OT) void cell_sort_one_kernel(
     int n, int m, int per, int ranges, SlabTable T, const uint32_t* __restrict__ keyI,
     const uint32_t* __restrict__ pidB, uint32_t* __restrict__ cs, uint32_t* __restrict__ skey,
@@ -405,7 +406,7 @@ __global__ __launch_bounds__(OT) void cell_sort_one_kernel(
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     auto cell_of = [&](uint32_t key) { return (int)(key & kCellKeyMask); };
     // this thread's sample of the keys: four neighbours share one of 256 places
-    const int sample = shares > 0 ? cell_of(keyI[(tid / 4) * (n / 4) / (OT / 4) * 4 + tid % 4]) : 0;
+    const int sample = SHARED ? cell_of(keyI[(tid / 4) * (n / 4) / (OT / 4) * 4 + tid % 4]) : 0;
     const uint4* const key4 = reinterpret_cast<const uint4*>(keyI);
     const int quads = n / 4;
     uint4 k[kOneLoads] = {};
@@ -418,7 +419,7 @@ __global__ __launch_bounds__(OT) void cell_sort_one_kernel(
     if (tid == 0) s_count = s_below = s_heavy = s_seen = 0u;
     const int block = xcd_tile(blockIdx.x, gridDim.x);
     int range = block, part = 0;
-    if (block >= ranges) {
+    if (SHARED && block >= ranges) {
         for (int r = tid; r < kOneGroups; r += OT) s_hist[r] = 0u;
         __syncthreads();
         atomicAdd(&s_hist[sample / per], 1u);
@@ -432,7 +433,7 @@ __global__ __launch_bounds__(OT) void cell_sort_one_kernel(
     int lo = range * per, hi = min(lo + per, m);  // this range of cells
     auto mine = [&](int c) { return c >= lo && c < hi; };
     __syncthreads();
-    if (shares > 0) {
+    if constexpr (SHARED) {
         const uint32_t found = (uint32_t)__popcll(__ballot(mine(sample)));
         if (lane == 0 && found) atomicAdd(&s_seen, found);
         __syncthreads();
@@ -653,7 +654,10 @@ hipError_t launch_cell_sort(sph_ctx* c, bool gather, hipStream_t s, bool counted
         const int groups = ranges + shares;
         const size_t lds = sizeof(uint32_t) * (2 * (size_t)per + 1 + 2 * one_list(n) +
                                                std::max(2 * one_list(n), heavy_words(n, gather && T.shift > 0)));
-        (gather ? cell_sort_one_kernel<true> : cell_sort_one_kernel<false>)<<<groups, OT, lds, s>>>(
+        const auto kernel =
+            shares > 0 ? (gather ? cell_sort_one_kernel<true, true> : cell_sort_one_kernel<false, true>)
+                       : (gather ? cell_sort_one_kernel<true, false> : cell_sort_one_kernel<false, false>);
+        kernel<<<groups, OT, lds, s>>>(
             n, m, per, ranges, T, b.keyI, b.pidB, b.cs, b.keyS[1], b.valS[1], b.posB, b.velB, b.posA, b.velA, b.pidA,
             tmp, rank);
         return hipGetLastError();
